@@ -253,17 +253,26 @@ struct DevGemm
 	int form = 1;          // one of GemmForm
 	double avg_steps = 0;  // mean k-steps per work item
 	double flops = 0;
-	// LDS-tiled form for the large tasks (both edges >= LDS_TASK_MIN): 64 x 64 tiles, one workgroup
-	// each (litems), the other tasks' 32 x 32 tiles (ritems) in the chosen form; used when use_lds
+	// LDS-tiled form (tile.hip): the 64 x 64 tiles of the large tasks (litems; both edges >= LDS_TASK_MIN),
+	// beside the other tasks' 32 x 32 tiles in the chosen form (ritems), or the tiles of every task (aitems)
 	WorkItem* litems = nullptr;
 	WorkItem* ritems = nullptr;
-	int nlitems = 0, nritems = 0;
-	bool use_lds = false;
-	void upload(const GemmBatch& b, hipStream_t s);
+	WorkItem* aitems = nullptr;
+	int nlitems = 0, nritems = 0, naitems = 0;
+	int tile_layout = -1;  // how the operands lie for the LDS-tiled form (tile_layout_of)
+	int use_lds = 0;       // one of TileUse
+	// tiles: with the item lists of the LDS-tiled form (plans that time their forms)
+	void upload(const GemmBatch& b, hipStream_t s, bool tiles = false);
 	void release();
 };
 constexpr int LDS_TILE = 64;       // output tile edge of the LDS-tiled form
-void split_lds_items(const GemmBatch& b, const std::vector<WorkItem>& it, std::vector<WorkItem>& lit, std::vector<WorkItem>& rit);
+enum TileUse { TILE_NONE = 0, TILE_LARGE = 1, TILE_ALL = 2 };
+// 64 x 64 tiles of the tasks with both edges at least min_edge (lit) and the items of the others (rit)
+void split_lds_items(const GemmBatch& b, const std::vector<WorkItem>& it, int min_edge, std::vector<WorkItem>& lit, std::vector<WorkItem>& rit);
+// 1: every A is stored k by k (sa_i 1), 0: every A is stored row by row (sa_k 1), in both every B is stored
+// k by k (sb_j 1) with its columns in one run (nci = N); -1: another layout, or an operand of 1 GiB or more
+// (the tiled form's offsets)
+int tile_layout_of(const GemmBatch& b);
 constexpr int LDS_TASK_MIN = 48;   // tasks with M and N at least this take the LDS-tiled form
 
 // Operand pointers in tasks/terms are byte offsets added to per-launch base pointers
@@ -272,6 +281,7 @@ struct GemmBases { const double* A; const double* B; double* C; };
 
 // kernel launchers (kernels.hip)
 void launch_grouped_gemm_f64(const DevGemm& g, GemmBases b, hipStream_t s);
+void launch_tile_gemm_f64(bool a_kmajor, const GemmTerm* terms, const WorkItem* items, int nitems, GemmBases b, hipStream_t s);
 void launch_grouped_gemm_split(const DevGemm& g, GemmBases b, hipStream_t s);
 void launch_plain_gemm_f64(const GemmTask& task, const GemmTerm& term, GemmBases b, hipStream_t s);
 void launch_permute(const double* src, double* dst, int ndim, const ct_long* dims, const int* perm, hipStream_t s);

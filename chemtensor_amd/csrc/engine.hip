@@ -63,12 +63,29 @@ std::vector<WorkItem> GemmBatch::work_items() const
 	return items;
 }
 
-// the LDS-tiled form's 64 x 64 tiles of the large tasks, and the other tasks' items (both empty when
-// no task is large). Workgroup i runs on XCD i mod 8, and each XCD has its own L2: the tiles of a
+int tile_layout_of(const GemmBatch& b)
+{
+	bool row = true, km = true;
+	for (const GemmTask& t : b.tasks) {
+		if (t.accumulate || t.nci != t.N || (int64_t)t.M * t.sc_i >= (int64_t)1 << 27) return -1;
+		for (int q = t.t0; q < t.t1; q++) {
+			const GemmTerm& m = b.terms[(size_t)q];
+			if (m.sb_j != 1 || m.sb_k < t.N) return -1;
+			row = row && m.sa_k == 1;
+			km = km && m.sa_i == 1 && m.sa_k >= t.M;
+			const int64_t ea = (int64_t)(t.M + 96) * m.sa_i + (int64_t)(m.K + 16) * m.sa_k, eb = (int64_t)(m.K + 16) * m.sb_k + t.N;
+			if (std::max(ea, eb) >= (int64_t)1 << 27) return -1;
+		}
+	}
+	return row ? 0 : km ? 1 : -1;
+}
+
+// the LDS-tiled form's 64 x 64 tiles of the tasks with both edges at least min_edge, and the other tasks'
+// items (both empty when there is no such task). Workgroup i runs on XCD i mod 8, and each XCD has its own L2: the tiles of a
 // task are cut into groups of up to 4 x 8 tiles (sharing A rows and B columns), the groups are
 // dealt to the eight XCDs by load (largest first), and the item order interleaves the XCDs' queues,
 // so a group's tiles run together on one XCD and fetch their operand panels into one L2.
-void split_lds_items(const GemmBatch& b, const std::vector<WorkItem>& it, std::vector<WorkItem>& lit, std::vector<WorkItem>& rit)
+void split_lds_items(const GemmBatch& b, const std::vector<WorkItem>& it, int min_edge, std::vector<WorkItem>& lit, std::vector<WorkItem>& rit)
 {
 	constexpr int NXCD = 8, GM = 4, GN = 8;
 	lit.clear();
@@ -85,7 +102,7 @@ void split_lds_items(const GemmBatch& b, const std::vector<WorkItem>& it, std::v
 	std::vector<int64_t> task_panels(b.tasks.size(), 0);
 	for (size_t ti = 0; ti < b.tasks.size(); ti++) {
 		const GemmTask& t = b.tasks[ti];
-		if (t.M < LDS_TASK_MIN || t.N < LDS_TASK_MIN || t.t1 <= t.t0) continue;
+		if (t.M < min_edge || t.N < min_edge) continue;
 		big[ti] = 1;
 		int64_t panels = 0;
 		for (int q = t.t0; q < t.t1; q++) panels += (b.terms[q].K + 15) / 16;
@@ -110,7 +127,7 @@ void split_lds_items(const GemmBatch& b, const std::vector<WorkItem>& it, std::v
 		const GemmTask& t = b.tasks[(size_t)g.task];
 		for (int mi = g.mi0; mi < g.mi1; mi++)
 			for (int ni = g.ni0; ni < g.ni1; ni++)
-				q[(size_t)x].push_back(WorkItem{ t, mi * LDS_TILE, ni * LDS_TILE, (int)tile_cost(t, task_panels[(size_t)g.task], mi, ni), g.task, b.terms[t.t0] });
+				q[(size_t)x].push_back(WorkItem{ t, mi * LDS_TILE, ni * LDS_TILE, (int)tile_cost(t, task_panels[(size_t)g.task], mi, ni), g.task, t.t1 > t.t0 ? b.terms[t.t0] : GemmTerm{} });
 	}
 	size_t longest = 0;
 	for (const auto& v : q) longest = std::max(longest, v.size());
@@ -120,7 +137,7 @@ void split_lds_items(const GemmBatch& b, const std::vector<WorkItem>& it, std::v
 	for (const WorkItem& w : it) if (!big[(size_t)w.task_index]) rit.push_back(w);
 }
 
-void DevGemm::upload(const GemmBatch& b, hipStream_t s)
+void DevGemm::upload(const GemmBatch& b, hipStream_t s, bool tiles)
 {
 	release();
 	const std::vector<WorkItem> it = b.work_items();
@@ -130,25 +147,32 @@ void DevGemm::upload(const GemmBatch& b, hipStream_t s)
 	flops = b.flops;
 	// the three tables in one allocation and one transfer (256-byte aligned parts)
 	std::vector<WorkItem> lit, rit;
-	split_lds_items(b, it, lit, rit);
+	std::vector<WorkItem> ait, none;
+	tile_layout = tiles ? tile_layout_of(b) : -1;
+	if (tiles) {
+		split_lds_items(b, it, LDS_TASK_MIN, lit, rit);
+		if (tile_layout >= 0) split_lds_items(b, it, 1, ait, none);
+	}
 	auto al = [](size_t n) { return (n + 255) / 256 * 256; };
 	const size_t n_tasks = b.tasks.size() * sizeof(GemmTask), n_terms = b.terms.size() * sizeof(GemmTerm), n_items = it.size() * sizeof(WorkItem);
-	const size_t n_lit = lit.size() * sizeof(WorkItem), n_rit = rit.size() * sizeof(WorkItem);
+	const size_t n_lit = lit.size() * sizeof(WorkItem), n_rit = rit.size() * sizeof(WorkItem), n_ait = ait.size() * sizeof(WorkItem);
 	const size_t o_terms = al(std::max<size_t>(n_tasks, 1)), o_items = o_terms + al(std::max<size_t>(n_terms, 1));
-	const size_t o_lit = o_items + al(std::max<size_t>(n_items, 1)), o_rit = o_lit + al(n_lit);
-	const size_t total = o_rit + std::max<size_t>(n_rit, 1);
+	const size_t o_lit = o_items + al(std::max<size_t>(n_items, 1)), o_rit = o_lit + al(n_lit), o_ait = o_rit + al(n_rit);
+	const size_t total = o_ait + std::max<size_t>(n_ait, 1);
 	buf = (char*)dev_alloc(total);
 	tasks = (GemmTask*)buf;
 	terms = (GemmTerm*)(buf + o_terms);
 	items = (WorkItem*)(buf + o_items);
 	litems = (WorkItem*)(buf + o_lit);
 	ritems = (WorkItem*)(buf + o_rit);
+	aitems = (WorkItem*)(buf + o_ait);
 	nlitems = (int)lit.size();
 	nritems = (int)rit.size();
-	use_lds = false;
-	const H2DPart parts[5] = { { b.tasks.data(), n_tasks, 0 }, { b.terms.data(), n_terms, o_terms }, { it.data(), n_items, o_items },
-		{ lit.data(), n_lit, o_lit }, { rit.data(), n_rit, o_rit } };
-	copy_h2d_parts(buf, parts, 5, o_rit + n_rit, s);
+	naitems = (int)ait.size();
+	use_lds = TILE_NONE;
+	const H2DPart parts[6] = { { b.tasks.data(), n_tasks, 0 }, { b.terms.data(), n_terms, o_terms }, { it.data(), n_items, o_items },
+		{ lit.data(), n_lit, o_lit }, { rit.data(), n_rit, o_rit }, { ait.data(), n_ait, o_ait } };
+	copy_h2d_parts(buf, parts, 6, o_ait + n_ait, s);
 	const int cap = num_compute_units() * 8;
 	grid = std::max(1, std::min((nitems + 3) / 4, cap));
 	// workgroup-level split of the k-step stream only pays for long streams
@@ -167,9 +191,9 @@ void DevGemm::release()
 {
 	dev_free(buf);
 	buf = nullptr;
-	tasks = nullptr; terms = nullptr; items = nullptr; litems = nullptr; ritems = nullptr;
-	ntasks = nterms = nitems = nlitems = nritems = 0;
-	use_lds = false;
+	tasks = nullptr; terms = nullptr; items = nullptr; litems = nullptr; ritems = nullptr; aitems = nullptr;
+	ntasks = nterms = nitems = nlitems = nritems = naitems = 0;
+	use_lds = TILE_NONE;
 }
 
 static void run_batch_plain(const GemmBatch& b, GemmBases bases, hipStream_t s)
@@ -903,29 +927,30 @@ int check_grouped_tables(const Meta& th, const Meta& W, const Meta& L, const Met
 	if (!check_batch(g.s1, th.nelem, R.nelem, g.t1_elems, &w1) || !once(w1)) return 1;
 	if (!check_batch(g.s2, W.nelem, g.t1_elems, g.t2_elems, &w2) || !once(w2)) return 2;
 	if (!check_batch(g.s3, L.nelem, g.t2_elems, th.nelem, &wy) || !once(wy)) return 3;
-	// the LDS-tiled split: every output entry of every task in exactly one 64 x 64 tile of a large
-	// task or one 32 x 32 item of another task
-	for (const GemmBatch* b : { &g.s1, &g.s2, &g.s3 }) {
-		const std::vector<WorkItem> it = b->work_items();
-		std::vector<WorkItem> lit, rit;
-		split_lds_items(*b, it, lit, rit);
-		if (lit.empty()) continue;
-		std::vector<int64_t> base(b->tasks.size() + 1, 0);
-		for (size_t ti = 0; ti < b->tasks.size(); ti++) base[ti + 1] = base[ti] + (int64_t)b->tasks[ti].M * b->tasks[ti].N;
-		std::vector<int> cover((size_t)base.back(), 0);
-		auto mark = [&](const WorkItem& w, int edge) {
-			const GemmTask& t = b->tasks[(size_t)w.task_index];
-			for (int i = w.m0; i < std::min(t.M, w.m0 + edge); i++)
-				for (int j = w.n0; j < std::min(t.N, w.n0 + edge); j++) cover[(size_t)(base[(size_t)w.task_index] + (int64_t)i * t.N + j)]++;
-		};
-		for (const WorkItem& w : lit) {
-			const GemmTask& t = b->tasks[(size_t)w.task_index];
-			if (t.M < LDS_TASK_MIN || t.N < LDS_TASK_MIN || w.first.K != b->terms[t.t0].K) return 8;
-			mark(w, LDS_TILE);
+	// the LDS-tiled splits: every output entry of every task in exactly one 64 x 64 tile of a large task or
+	// one 32 x 32 item of another task
+	for (const GemmBatch* b : { &g.s1, &g.s2, &g.s3 })
+		for (const int min_edge : { LDS_TASK_MIN, 1 }) {
+			const std::vector<WorkItem> it = b->work_items();
+			std::vector<WorkItem> lit, rit;
+			split_lds_items(*b, it, min_edge, lit, rit);
+			if (lit.empty()) continue;
+			std::vector<int64_t> base(b->tasks.size() + 1, 0);
+			for (size_t ti = 0; ti < b->tasks.size(); ti++) base[ti + 1] = base[ti] + (int64_t)b->tasks[ti].M * b->tasks[ti].N;
+			std::vector<int> cover((size_t)base.back(), 0);
+			auto mark = [&](const WorkItem& w, int edge) {
+				const GemmTask& t = b->tasks[(size_t)w.task_index];
+				for (int i = w.m0; i < std::min(t.M, w.m0 + edge); i++)
+					for (int j = w.n0; j < std::min(t.N, w.n0 + edge); j++) cover[(size_t)(base[(size_t)w.task_index] + (int64_t)i * t.N + j)]++;
+			};
+			for (const WorkItem& w : lit) {
+				const GemmTask& t = b->tasks[(size_t)w.task_index];
+				if (t.M < min_edge || t.N < min_edge || (t.t1 > t.t0 && w.first.K != b->terms[t.t0].K)) return 8;
+				mark(w, LDS_TILE);
+			}
+			for (const WorkItem& w : rit) mark(w, TILE);
+			if (!once(cover)) return 8;
 		}
-		for (const WorkItem& w : rit) mark(w, TILE);
-		if (!once(cover)) return 8;
-	}
 	const WApplyHost& wa = g.wa;
 	if (wa.kmax <= WA_KMAX) {
 		std::vector<int> ws((size_t)g.t2_elems, 0);
@@ -991,9 +1016,10 @@ static void build_grouped(MatvecPlan& p, bool lean)
 	m2.nelem = g.t2_elems;
 	p.interm.emplace_back(std::move(m1));
 	p.interm.emplace_back(std::move(m2));
-	p.stage[0].upload(g.s1, p.stream);
-	p.stage[1].upload(g.s2, p.stream);
-	p.stage[2].upload(g.s3, p.stream);
+	const bool tiles = p.mode == CT_MATVEC_GROUPED_FP64 && !lean;
+	p.stage[0].upload(g.s1, p.stream, tiles);
+	p.stage[1].upload(g.s2, p.stream, tiles);
+	p.stage[2].upload(g.s3, p.stream, tiles);
 	for (int i = 0; i < 3; i++) p.stage_bytes[i] = g.stage_bytes[i];
 	p.stage_flops[0] = g.s1.flops;
 	p.stage_flops[1] = g.s2.flops;
@@ -1138,15 +1164,21 @@ void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, 
 			if (ms < best) { best = ms; best_form = f; }
 		}
 		g.form = best_form;
-		// the large tasks on the LDS-tiled form, the rest on the best form (CT_GEMM_LDS=0|1 overrides)
-		if (g.nlitems > 0) {
-			g.use_lds = true;
-			const float ms = time3([&] { launch_grouped_gemm_f64(g, b, s); });
-			g.use_lds = ms < best;
-			if (g.use_lds) best = ms;
+		// the large tasks on the LDS-tiled form and the rest on the best form, or every task on the LDS-tiled
+		// form (CT_GEMM_LDS=0|1: never / the faster of the two, whatever the others take)
+		if (g.nlitems > 0 || g.naitems > 0) {
+			float tile_best = 1e30f;
+			int tile_use = TILE_NONE;
+			for (const int use : { TILE_LARGE, TILE_ALL }) {
+				if (use == TILE_LARGE ? g.nlitems == 0 : g.naitems == 0) continue;
+				g.use_lds = use;
+				const float ms = time3([&] { launch_grouped_gemm_f64(g, b, s); });
+				if (ms < tile_best) { tile_best = ms; tile_use = use; }
+			}
 			const char* force = getenv("CT_GEMM_LDS");
-			if (force && force[0] == '0') g.use_lds = false;
-			if (force && force[0] == '1') g.use_lds = true;
+			const bool use = force && force[0] == '0' ? false : force && force[0] == '1' ? true : tile_best < best;
+			g.use_lds = use ? tile_use : TILE_NONE;
+			if (use && tile_best < best) best = tile_best;
 		}
 		if (st == 0) best1 = best;
 		if (st == 1) best2 = best;

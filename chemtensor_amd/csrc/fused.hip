@@ -605,9 +605,9 @@ BatchPlan* build_batch_plan(std::vector<BatchInput>& in, hipStream_t s, bool tun
 	b->t1 = (double*)dev_alloc((size_t)std::max<int64_t>(g.t1_elems, 1) * sizeof(double));
 	b->t2 = (double*)dev_alloc((size_t)std::max<int64_t>(g.t2_elems, 1) * sizeof(double));
 	if (!tune && !split) b->flops = g.s1.flops + g.s2.flops + g.s3.flops;   // executed count (no replanning of the reference sequence)
-	b->stage[0].upload(g.s1, s);
-	b->stage[1].upload(g.s2, s);
-	b->stage[2].upload(g.s3, s);
+	b->stage[0].upload(g.s1, s, tune);
+	b->stage[1].upload(g.s2, s, tune);
+	b->stage[2].upload(g.s3, s, tune);
 	b->stage_bases[0] = GemmBases{ nullptr, b->r, b->t1 };
 	b->stage_bases[1] = GemmBases{ b->w, b->t1, b->t2 };
 	b->stage_bases[2] = GemmBases{ b->l, b->t2, nullptr };

@@ -1,0 +1,48 @@
+"""The LDS-tiled GEMM form of the grouped matvec (64 x 64 tiles, CT_GEMM_LDS=1) at the edges of its tiles,
+k-panels and 16 x 16 sub-tiles, against a dense FP64 contraction."""
+
+import sys
+
+import numpy as np
+import pytest
+
+import chemtensor_amd as ct
+
+pytestmark = pytest.mark.gpu
+
+
+def dense_problem(da, db, d, D, seed):
+    """One sector on every axis: stage 1 is a (da d) x (D db) product with K = db, stage 3 da x (d db) with K = da D."""
+    rng = np.random.default_rng(seed)
+    z = lambda n: np.zeros(n, dtype=np.int32)
+    shapes = [(da, d, db), (D, d, d, D), (1, da, D, da), (db, D, db, 1)]
+    dirs = [[1, 1, -1], [1, 1, -1, -1], [1, -1, -1, 1], [1, 1, -1, -1]]
+    ts, vs = [], []
+    for s, ad in zip(shapes, dirs):
+        t = ct.HostTensor.zeros(s, ad, [z(n) for n in s])
+        v = rng.standard_normal(s)
+        t.deserialize(v.reshape(-1))
+        ts.append(t)
+        vs.append(v)
+    th, w, l, r = vs
+    t1 = np.tensordot(th, r[..., 0], axes=(2, 0))                       # a p n c
+    t2 = np.tensordot(w, t1, axes=([2, 3], [1, 2]))                     # m q a c
+    return ts, np.einsum("amx,mqac->xqc", l[0], t2, optimize=True).reshape(-1)
+
+
+@pytest.mark.parametrize("da,db,d,D", [(1, 1, 1, 1), (1, 3, 2, 2), (15, 17, 1, 1), (16, 16, 2, 1), (17, 15, 3, 1), (33, 64, 1, 2), (48, 5, 1, 3),
+                                       (63, 65, 2, 1), (64, 32, 1, 1), (65, 33, 2, 2), (130, 129, 1, 2), (3, 200, 4, 5), (200, 3, 4, 5)])
+def test_tile_form_edges(da, db, d, D, monkeypatch):
+    monkeypatch.setenv("CT_GEMM_LDS", "1")
+    monkeypatch.setenv("CT_STAGE12", "separate")
+    ts, want = dense_problem(da, db, d, D, 100 * da + db)
+    plan = ct.MatvecPlan(*ts, ct.GROUPED_FP64)
+    forms = plan.forms()[0]
+    print("case", da, db, d, D, "forms", forms, flush=True)
+    sys.stdout.flush()
+    assert forms[0] == 6 and forms[2] == 6
+    x, y = ct.DeviceArray.from_numpy(ts[0].serialize()), ct.DeviceArray(plan.dim)
+    plan.apply(x, y)
+    plan.synchronize()
+    # three chained FP64 products of at most 1000 terms: 2e-16 sqrt(1000) each way
+    assert np.linalg.norm(y.numpy() - want) <= 2e-14 * np.linalg.norm(want)
