@@ -281,7 +281,10 @@ struct GemmBases { const double* A; const double* B; double* C; };
 
 // kernel launchers (kernels.hip)
 void launch_grouped_gemm_f64(const DevGemm& g, GemmBases b, hipStream_t s);
-void launch_tile_gemm_f64(bool a_kmajor, const GemmTerm* terms, const WorkItem* items, int nitems, GemmBases b, hipStream_t s);
+// udot (optional, nitems entries): per tile, its entries times x at their indices in the result vector (a
+// task's first index is its pad field)
+void launch_tile_gemm_f64(bool a_kmajor, const GemmTerm* terms, const WorkItem* items, int nitems, GemmBases b, hipStream_t s,
+	const double* x = nullptr, double* udot = nullptr);
 void launch_grouped_gemm_split(const DevGemm& g, GemmBases b, hipStream_t s);
 void launch_plain_gemm_f64(const GemmTask& task, const GemmTerm& term, GemmBases b, hipStream_t s);
 void launch_permute(const double* src, double* dst, int ndim, const ct_long* dims, const int* perm, hipStream_t s);
@@ -459,6 +462,7 @@ void launch_pair_matvec(const PairPlan& pp, const double* x, const double* r, co
 // the matvec with the Lanczos alpha partials of <y, x> from its partial-sum launch: dpart[0 .. G),
 // G = pair_dot_partials(pp)
 int pair_dot_partials(const PairPlan& pp);
+void launch_pair_reduce_dot(const PairPlan& pp, const double* x, double* y, double* dpart, hipStream_t s);
 void launch_pair_matvec_dot(const PairPlan& pp, const double* x, const double* r, const double* l, double* y, double* dpart, hipStream_t s);
 // one deferred-normalisation Lanczos step on a sector-pair plan after launch_pair_units(.., dpart):
 // beta from npart (the previous step's workgroup partials), alpha from the unit partials dpart, y
@@ -521,6 +525,29 @@ int lanczos_eigensystem(LanczosWork& lw, int64_t n, hipStream_t s, const DevMatv
 	int maxiter, int numeig, double* lambda, double* u, bool use_graph = false, bool sync_stop = false, const DevMatvecDot* matvec_dot = nullptr,
 	bool deferred = false);
 
+// Stage 3 with the k range of every y block cut into slots of about 'panels' k-panels: the slots are tasks
+// of the LDS-tiled form writing partial blocks, which the partial-sum launch of the sector-pair form adds in
+// slot order.
+struct Stage3Split
+{
+	DevGemm g;
+	PairPlan sum;          // partial blocks and reduction items (nunits: tiles)
+	bool ok = false;       // the tables are there
+	bool use = false;      // the faster of the two ways to run stage 3
+	bool use_lanczos = false;   // the faster one in a Lanczos step, whose update adds the slots itself
+	void build(const GemmBatch& s3, hipStream_t s);
+	void release();
+};
+// the slots' tasks (C: element offsets of the partial blocks, pad: the block's first index in y) and the
+// reduction items of a stage-3 batch; false where the tiled form does not apply
+bool split_stage3(const GemmBatch& s3, int panels, GemmBatch& out, std::vector<PrRed>& red, int64_t& part_elems);
+// y partial blocks of stage 3, with the alpha partials <y, x> per tile when udot is given
+void launch_stage3_units(const Stage3Split& sp, GemmBases b, hipStream_t s, const double* x = nullptr, double* udot = nullptr);
+
+// a Lanczos step on the split stage 3 has one launch less than on the tasks (the step adds the slots, the
+// tiles write the alpha partials): worth this much (ms)
+constexpr float LZ_SAVED_MS = 0.006f;
+
 struct MatvecPlan
 {
 	int mode = 1;
@@ -534,6 +561,7 @@ struct MatvecPlan
 	WApply wapply;                              // column-stream form of stage 2
 	bool use_wapply = false;
 	bool use_f12 = false;                       // stages 1 and 2 fused (no T1 in HBM)
+	Stage3Split split3;
 	// fused form: one launch
 	FusedPlan fused;
 	// sector-pair form: one unit launch and one reduction launch
@@ -578,11 +606,14 @@ void merge_grouped_tables(GroupedTables& dst, const GroupedTables& src, int64_t 
 void validate_matvec_operands(const Meta& theta, const Meta& w, const Meta& l, const Meta& r);
 // time every launch form of each grouped stage (and the column-stream stage 2 when available) and
 // keep the fastest; sets *use_wapply
-void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, bool* use_wapply, bool* use_f12, int64_t nx, hipStream_t s,
-	float (*tuned_ms)[GEMM_NUM_FORMS]);
+void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, bool* use_wapply, bool* use_f12, Stage3Split* split3, int64_t nx,
+	hipStream_t s, float (*tuned_ms)[GEMM_NUM_FORMS]);
 // one grouped matvec: stage 1, stage 2 (MFMA tiles or column stream), stage 3
-void launch_grouped_stages(const DevGemm* stage, const GemmBases* bases, const WApply* wa, bool use_wapply, bool use_f12, const double* x, double* y,
-	hipStream_t s, hipEvent_t* ev);
+void launch_grouped_stages(const DevGemm* stage, const GemmBases* bases, const WApply* wa, bool use_wapply, bool use_f12, const Stage3Split* split3,
+	const double* x, double* y, hipStream_t s, hipEvent_t* ev);
+
+// stages 1 and 2 and the tiles of the split stage 3 with the alpha partials <y, x> (split3.sum.nunits)
+void launch_grouped_units(const MatvecPlan& p, const double* x, double* udot);
 
 // FP64 flops of the reference's unfused operation sequence: sum of 2 m n k over its GEMM calls
 double reference_flops(const Meta& th, const Meta& w, const Meta& l, const Meta& r);
@@ -627,6 +658,7 @@ struct BatchPlan
 	WApply wapply;
 	bool use_wapply = false;
 	bool use_f12 = false;
+	Stage3Split split3;
 	double* t1 = nullptr;
 	double* t2 = nullptr;
 	bool use_fused = false;                     // the faster of the two forms, timed at plan creation

@@ -77,7 +77,7 @@ int tile_layout_of(const GemmBatch& b)
 			if (std::max(ea, eb) >= (int64_t)1 << 27) return -1;
 		}
 	}
-	return row ? 0 : km ? 1 : -1;
+	return km ? 1 : row ? 0 : -1;
 }
 
 // the LDS-tiled form's 64 x 64 tiles of the tasks with both edges at least min_edge, and the other tasks'
@@ -185,6 +185,86 @@ void DevGemm::upload(const GemmBatch& b, hipStream_t s, bool tiles)
 	const double avg = nitems ? steps / nitems : 0;
 	form = (avg > 8.0) ? GEMM_WG_CHUNK : GEMM_WAVE_STREAM;
 	avg_steps = avg;
+}
+
+// k-panels of a term in the LDS-tiled form
+static int64_t term_panels(const GemmTerm& m) { return (m.K + 15) / 16; }
+
+bool split_stage3(const GemmBatch& s3, int panels, GemmBatch& out, std::vector<PrRed>& red, int64_t& part_elems)
+{
+	if (tile_layout_of(s3) != 1) return false;
+	part_elems = 0;
+	for (const GemmTask& t : s3.tasks) {
+		const int64_t y0 = (int64_t)((intptr_t)t.C / (intptr_t)sizeof(double)), size = (int64_t)t.M * t.N;
+		if (t.sc_i != t.N || y0 + size > INT32_MAX || size > INT32_MAX) return false;
+		int64_t total = 0;
+		for (int q = t.t0; q < t.t1; q++) total += term_panels(s3.terms[(size_t)q]);
+		const int64_t nslots = total > 0 ? std::max<int64_t>(1, (total + panels / 2) / panels) : 0;
+		// slot i: panels [total i / nslots, total (i + 1) / nslots) of the task's terms in order
+		int q = t.t0;
+		int64_t q0 = 0;   // panels before term q
+		for (int64_t i = 0; i < nslots; i++) {
+			const int64_t p0 = total * i / nslots, p1 = total * (i + 1) / nslots;
+			out.add_task(off_ptr_mut(part_elems + i * size), t.M, t.N, t.N, t.N, 0, false);
+			out.tasks.back().pad = (int32_t)y0;
+			while (q < t.t1 && q0 < p1) {
+				const GemmTerm& m = s3.terms[(size_t)q];
+				const int64_t np = term_panels(m);
+				const int64_t a = std::max(p0, q0) - q0, b = std::min(p1, q0 + np) - q0;
+				if (b > a) {
+					const int64_t k0 = 16 * a, k1 = std::min<int64_t>(16 * b, m.K);
+					out.add_term(m.A + k0 * m.sa_k, m.B + k0 * m.sb_k, (int)(k1 - k0), m.sa_i, m.sa_k, m.sb_k, m.sb_j, m.sb_batch);
+				}
+				if (q0 + np > p1) break;
+				q0 += np;
+				q++;
+			}
+		}
+		for (int64_t e0 = 0; e0 < size; e0 += 64)
+			red.push_back(PrRed{ y0 + e0, nslots ? part_elems + e0 : 0, (int32_t)std::min<int64_t>(64, size - e0), (int32_t)size, (int32_t)nslots, 0 });
+		part_elems += nslots * size;
+	}
+	return true;
+}
+
+void Stage3Split::build(const GemmBatch& s3, hipStream_t s)
+{
+	release();
+	// three tiles per compute unit where the work allows it: slots of at least 6 panels (XXZ bond of 515
+	// states, units and sums: 6 panels 24.6 us, 8 26.8, 16 29.0; 4 panels 26.4) and of at most 24 (molecular
+	// operator, 20 orbitals: 24 panels 205 us, 16 212, 8 240), beyond which only the partial blocks shrink
+	int64_t total = 0;
+	for (const GemmTask& t : s3.tasks) {
+		int64_t tp = 0;
+		for (int q = t.t0; q < t.t1; q++) tp += term_panels(s3.terms[(size_t)q]);
+		total += tp * ((t.M + LDS_TILE - 1) / LDS_TILE) * ((t.N + LDS_TILE - 1) / LDS_TILE);
+	}
+	const int panels = (int)std::min<int64_t>(24, std::max<int64_t>(6, total / (3 * num_compute_units())));
+	GemmBatch b;
+	std::vector<PrRed> red;
+	int64_t elems = 0;
+	if (!split_stage3(s3, panels, b, red, elems)) return;
+	g.upload(b, s, true);
+	sum.red = (PrRed*)dev_alloc(std::max<size_t>(1, red.size()) * sizeof(PrRed));
+	copy_h2d_async(sum.red, red.data(), red.size() * sizeof(PrRed), s);
+	sum.nred = (int)red.size();
+	sum.part = (double*)dev_alloc((size_t)std::max<int64_t>(1, elems) * sizeof(double));
+	sum.part_elems = elems;
+	sum.nunits = g.naitems;
+	ok = true;
+}
+
+void Stage3Split::release()
+{
+	g.release();
+	sum.release();
+	ok = use = use_lanczos = false;
+}
+
+void launch_stage3_units(const Stage3Split& sp, GemmBases b, hipStream_t s, const double* x, double* udot)
+{
+	b.C = sp.sum.part;
+	launch_tile_gemm_f64(true, sp.g.terms, sp.g.aitems, sp.g.naitems, b, s, x, udot);
 }
 
 void DevGemm::release()
@@ -575,6 +655,7 @@ DevTensor dev_split_axis(const DevTensor& t, int i_ax, const ct_long* nd2, const
 MatvecPlan::~MatvecPlan()
 {
 	for (int i = 0; i < 3; i++) stage[i].release();
+	split3.release();
 	wapply.release();
 	fused.release();
 	pair.release();
@@ -951,6 +1032,24 @@ int check_grouped_tables(const Meta& th, const Meta& W, const Meta& L, const Met
 			for (const WorkItem& w : rit) mark(w, TILE);
 			if (!once(cover)) return 8;
 		}
+	// the split stage 3: every partial entry written once from operands in range, every y entry the sum of its
+	// block's slots, every k of a block in one of them
+	for (const int panels : { 1, 6 }) {
+		GemmBatch sp;
+		std::vector<PrRed> red;
+		int64_t elems = 0;
+		if (!split_stage3(g.s3, panels, sp, red, elems)) continue;
+		std::vector<int> wp((size_t)elems, 0), wr((size_t)th.nelem, 0);
+		if (!check_batch(sp, L.nelem, g.t2_elems, elems, &wp) || !once(wp)) return 9;
+		int64_t k0 = 0, k1 = 0;
+		for (const GemmTask& t : g.s3.tasks) for (int q = t.t0; q < t.t1; q++) k0 += (int64_t)t.M * t.N * g.s3.terms[(size_t)q].K;
+		for (const GemmTask& t : sp.tasks) for (int q = t.t0; q < t.t1; q++) k1 += (int64_t)t.M * t.N * sp.terms[(size_t)q].K;
+		for (const PrRed& r : red) {
+			if (r.n < 1 || r.n > 64 || r.y < 0 || r.y + r.n > th.nelem || (r.nslots > 0 && r.p + (int64_t)(r.nslots - 1) * r.size + r.n > elems)) return 9;
+			for (int e = 0; e < r.n; e++) wr[(size_t)(r.y + e)]++;
+		}
+		if (k0 != k1 || !once(wr)) return 9;
+	}
 	const WApplyHost& wa = g.wa;
 	if (wa.kmax <= WA_KMAX) {
 		std::vector<int> ws((size_t)g.t2_elems, 0);
@@ -1021,6 +1120,7 @@ static void build_grouped(MatvecPlan& p, bool lean)
 	p.stage[1].upload(g.s2, p.stream, tiles);
 	p.stage[2].upload(g.s3, p.stream, tiles);
 	for (int i = 0; i < 3; i++) p.stage_bytes[i] = g.stage_bytes[i];
+	if (tiles) p.split3.build(g.s3, p.stream);
 	p.stage_flops[0] = g.s1.flops;
 	p.stage_flops[1] = g.s2.flops;
 	p.stage_flops[2] = g.s3.flops;
@@ -1130,7 +1230,7 @@ static void build_plain(MatvecPlan& p)
 // warm-up and three timed launches, HIP events on the plan stream); the fastest form is kept.
 // time every launch form of each grouped stage on the plan's own descriptors (x = 1, y scratch)
 // and keep the fastest; stage 2 also tries the column-stream form
-void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, bool* use_wapply, bool* use_f12, int64_t nx, hipStream_t s,
+void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, bool* use_wapply, bool* use_f12, Stage3Split* split3, int64_t nx, hipStream_t s,
 	float (*tuned_ms)[GEMM_NUM_FORMS])
 {
 	double* x = (double*)dev_alloc((size_t)std::max<int64_t>(nx, 1) * sizeof(double));
@@ -1182,6 +1282,15 @@ void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, 
 		}
 		if (st == 0) best1 = best;
 		if (st == 1) best2 = best;
+		if (st == 2 && split3 && split3->ok) {
+			const float ms = time3([&] { launch_stage3_units(*split3, b, s); launch_pair_reduce(split3->sum, y, s); });
+			split3->use = ms < best;
+			split3->use_lanczos = split3->use || ms - best < LZ_SAVED_MS;
+			// CT_STAGE3=split|tasks overrides the timing-based choice
+			const char* force = getenv("CT_STAGE3");
+			if (force && strcmp(force, "tasks") == 0) split3->use = split3->use_lanczos = false;
+			if (force && strcmp(force, "split") == 0) split3->use = split3->use_lanczos = true;
+		}
 	}
 	if (use_wapply) {
 		*use_wapply = false;
@@ -1213,14 +1322,14 @@ void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, 
 	dev_free(y);
 }
 
-void launch_grouped_stages(const DevGemm* stage, const GemmBases* bases, const WApply* wa, bool use_wapply, bool use_f12, const double* x, double* y,
-	hipStream_t s, hipEvent_t* ev)
+// launch stages 1 and 2 of a grouped matvec
+static void launch_stages12(const DevGemm* stage, const GemmBases* bases, const WApply* wa, bool use_wapply, bool use_f12, const double* x, hipStream_t s,
+	hipEvent_t* ev)
 {
 	const bool f12 = use_f12 && wa && wa->f12_ok;
-	for (int st = 0; st < 3; st++) {
+	for (int st = 0; st < 2; st++) {
 		GemmBases b = bases[st];
 		if (st == 0) b.A = x;
-		if (st == 2) b.C = y;
 		if (st == 0 && f12) launch_f12(*wa, x, b.B, bases[1].C, s);
 		else if (st == 1 && f12) { /* done by the fused launch */ }
 		else if (st == 1 && use_wapply && wa && wa->ok) launch_wapply(*wa, b.B, b.C, s);
@@ -1229,9 +1338,29 @@ void launch_grouped_stages(const DevGemm* stage, const GemmBases* bases, const W
 	}
 }
 
+void launch_grouped_units(const MatvecPlan& p, const double* x, double* udot)
+{
+	launch_stages12(p.stage, p.stage_bases, &p.wapply, p.use_wapply, p.use_f12, x, p.stream, nullptr);
+	launch_stage3_units(p.split3, p.stage_bases[2], p.stream, x, udot);
+}
+
+void launch_grouped_stages(const DevGemm* stage, const GemmBases* bases, const WApply* wa, bool use_wapply, bool use_f12, const Stage3Split* split3,
+	const double* x, double* y, hipStream_t s, hipEvent_t* ev)
+{
+	launch_stages12(stage, bases, wa, use_wapply, use_f12, x, s, ev);
+	GemmBases b = bases[2];
+	b.C = y;
+	if (split3 && split3->use) {
+		launch_stage3_units(*split3, b, s);
+		launch_pair_reduce(split3->sum, y, s);
+	}
+	else launch_grouped_gemm_f64(stage[2], b, s);
+	if (ev) CTG_HIP(hipEventRecord(ev[3], s));
+}
+
 static void autotune_stages(MatvecPlan& p)
 {
-	autotune_grouped(p.stage, p.stage_bases, &p.wapply, &p.use_wapply, &p.use_f12, p.theta_meta.nelem, p.stream, p.tuned_ms);
+	autotune_grouped(p.stage, p.stage_bases, &p.wapply, &p.use_wapply, &p.use_f12, &p.split3, p.theta_meta.nelem, p.stream, p.tuned_ms);
 	if (p.use_f12 && p.wapply.f12_ok) {
 		// one launch for stages 1 and 2: theta, R and W in, T2 out (T1 never written)
 		const double t1 = (double)p.interm[0].meta.nelem;
@@ -1384,6 +1513,10 @@ float matvec_stage_time(MatvecPlan& p, int stage, const double* x, double* y, in
 		}
 		else if (stage < 2 && p.use_f12 && p.wapply.f12_ok) { if (stage == 0) launch_f12(p.wapply, x, b.B, p.stage_bases[1].C, s); }
 		else if (stage == 1 && p.use_wapply && p.wapply.ok) launch_wapply(p.wapply, b.B, b.C, s);
+		else if (stage == 2 && p.split3.use) {
+			launch_stage3_units(p.split3, b, s);
+			launch_pair_reduce(p.split3.sum, y, s);
+		}
 		else launch_grouped_gemm_f64(p.stage[stage], b, s);
 	};
 	launch();
@@ -1427,7 +1560,7 @@ void matvec_apply(MatvecPlan& p, const double* x, double* y, float* stage_ms)
 			if (stage_ms) CTG_HIP(hipEventRecord(p.ev[st + 1], s));
 		}
 	}
-	else launch_grouped_stages(p.stage, p.stage_bases, &p.wapply, p.use_wapply, p.use_f12, x, y, s, stage_ms ? p.ev : nullptr);
+	else launch_grouped_stages(p.stage, p.stage_bases, &p.wapply, p.use_wapply, p.use_f12, &p.split3, x, y, s, stage_ms ? p.ev : nullptr);
 	if (stage_ms) {
 		CTG_HIP(hipEventSynchronize(p.ev[3]));
 		for (int st = 0; st < 3; st++) CTG_HIP(hipEventElapsedTime(&stage_ms[st], p.ev[st], p.ev[st + 1]));

@@ -479,9 +479,23 @@ int lanczos_ground_state(MatvecPlan& p, const double* vstart, int maxiter, doubl
 			};
 		}
 	}
+	// grouped plans with the split stage 3: the same two parts, behind stages 1 and 2
+	else if (p.mode == CT_MATVEC_GROUPED_FP64 && p.split3.use_lanczos) {
+		mvd.partials = pair_dot_partials(p.split3.sum);
+		mvd.apply = [&p](const double* x, double* y, double* part) {
+			launch_grouped_units(p, x, nullptr);
+			launch_pair_reduce_dot(p.split3.sum, x, y, part, p.stream);
+		};
+		mvd.step_partials = pair_step_partials(p.split3.sum);
+		mvd.units = [&p](const double* x, double* part) { launch_grouped_units(p, x, part); };
+		mvd.step = [&p](const double* uj, double* unext, double* vj_out, const double* vjm1, int j, int maxiter, const double* dpart,
+			const double* npart, double thresh, double* npart_out, double* scal) {
+			launch_pair_lz_step(p.split3.sum, uj, unext, vj_out, vjm1, j, maxiter, dpart, npart, thresh, npart_out, scal, p.stream);
+		};
+	}
 	return lanczos_eigensystem(p.lz, p.theta_meta.nelem, p.stream,
 		[&p](const double* x, double* y) { matvec_apply(p, x, y, nullptr); }, vstart, maxiter, 1, lambda, u, graph, false,
-		p.mode == CT_MATVEC_PAIR_FP64 ? &mvd : nullptr, lanczos_deferred());
+		mvd.partials > 0 ? &mvd : nullptr, lanczos_deferred());
 }
 
 //________________________________________________________________________________________________________________________

@@ -1347,12 +1347,17 @@ void launch_pair_lz_step(const PairPlan& pp, const double* uj, double* unext, do
 	CTG_HIP(hipGetLastError());
 }
 
-void launch_pair_matvec_dot(const PairPlan& pp, const double* x, const double* r, const double* l, double* y, double* dpart, hipStream_t s)
+void launch_pair_reduce_dot(const PairPlan& pp, const double* x, double* y, double* dpart, hipStream_t s)
 {
-	launch_pair_units(pp, x, r, l, s);
 	hipLaunchKernelGGL(k_pair_reduce_dot, dim3((unsigned)pair_dot_partials(pp)), dim3(256), 0, s, (const PrRed*)pp.red, pp.nred, (const double*)pp.part,
 		y, x, dpart);
 	CTG_HIP(hipGetLastError());
+}
+
+void launch_pair_matvec_dot(const PairPlan& pp, const double* x, const double* r, const double* l, double* y, double* dpart, hipStream_t s)
+{
+	launch_pair_units(pp, x, r, l, s);
+	launch_pair_reduce_dot(pp, x, y, dpart, s);
 }
 
 //________________________________________________________________________________________________________________________

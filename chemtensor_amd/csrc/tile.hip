@@ -71,8 +71,11 @@ struct TilePanel { double2_t a[2], b[2]; };
 // per CU; a double buffer with one barrier per panel allows four: 172 us against 160 us for stage 1 of a
 // Hubbard bond of 2000 states, 6.3 GFLOP).
 // AK: A is stored k by k (sa_i 1), else row by row (sa_k 1); B is stored k by k (sb_j 1).
-template <bool AK>
-__global__ __launch_bounds__(256, 4) void k_tile_gemm_f64(const GemmTerm* __restrict__ terms, const WorkItem* __restrict__ items, GemmBases bs)
+// DOT: udot[tile] = the sum of its entries times x at their indices in the result vector (butterfly within
+// each wavefront, then the four wavefronts in order).
+template <bool AK, bool DOT>
+__global__ __launch_bounds__(256, 4) void k_tile_gemm_f64(const GemmTerm* __restrict__ terms, const WorkItem* __restrict__ items, GemmBases bs,
+	const double* __restrict__ x, double* __restrict__ udot)
 {
 	__shared__ __attribute__((aligned(16))) double sa[TPANEL];
 	__shared__ __attribute__((aligned(16))) double sb[TPANEL];
@@ -233,6 +236,9 @@ __global__ __launch_bounds__(256, 4) void k_tile_gemm_f64(const GemmTerm* __rest
 	const int sc_i = it->task.sc_i;
 	const TileOperand oc = { (uint64_t)(uintptr_t)rebase(bs.C, it->task.C), 8 * ((M - 1) * sc_i + N) };
 	const __amdgpu_buffer_rsrc_t rc = oc.rsrc();
+	const TileOperand ox = { DOT ? (uint64_t)(uintptr_t)(x + it->task.pad) : 0, DOT ? oc.bytes : 0 };
+	const __amdgpu_buffer_rsrc_t rx = ox.rsrc();
+	double dot = 0;
 	#pragma unroll
 	for (int sub = 0; sub < 4; sub++) {
 		const int mi = sub >> 1, ni = sub & 1;
@@ -241,16 +247,31 @@ __global__ __launch_bounds__(256, 4) void k_tile_gemm_f64(const GemmTerm* __rest
 		const int col = n0 + 16 * (cb0 + ni) + i16, row0 = m0 + 16 * (rb0 + mi) + kq;
 		const int off = col < N ? 8 * (row0 * sc_i + col) : TILE_OOB;
 		#pragma unroll
-		for (int rr = 0; rr < 4; rr++)
-			__builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(uint2_t, (double)acc[rr]), rc, row0 + 4 * rr < M ? off + 32 * rr * sc_i : TILE_OOB, 0, 0);
+		for (int rr = 0; rr < 4; rr++) {
+			const int o = row0 + 4 * rr < M ? off + 32 * rr * sc_i : TILE_OOB;
+			__builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(uint2_t, (double)acc[rr]), rc, o, 0, 0);
+			if constexpr (DOT) dot += acc[rr] * __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rx, o, 0, 0));
+		}
+	}
+	if constexpr (DOT) {
+		#pragma unroll
+		for (int o = 32; o > 0; o >>= 1) dot += __shfl_xor(dot, o, 64);
+		__syncthreads();
+		if (lane == 0) sa[wave] = dot;
+		__syncthreads();
+		if (tid == 0) udot[blockIdx.x] = (sa[0] + sa[1]) + (sa[2] + sa[3]);
 	}
 }
 
-void launch_tile_gemm_f64(bool a_kmajor, const GemmTerm* terms, const WorkItem* items, int nitems, GemmBases b, hipStream_t s)
+void launch_tile_gemm_f64(bool a_kmajor, const GemmTerm* terms, const WorkItem* items, int nitems, GemmBases b, hipStream_t s, const double* x,
+	double* udot)
 {
 	if (nitems == 0) return;
-	if (a_kmajor) hipLaunchKernelGGL(k_tile_gemm_f64<true>, dim3((unsigned)nitems), dim3(256), 0, s, terms, items, b);
-	else hipLaunchKernelGGL(k_tile_gemm_f64<false>, dim3((unsigned)nitems), dim3(256), 0, s, terms, items, b);
+	const dim3 grid((unsigned)nitems), block(256);
+	if (udot && a_kmajor) hipLaunchKernelGGL((k_tile_gemm_f64<true, true>), grid, block, 0, s, terms, items, b, x, udot);
+	else if (udot) throw HipError{ hipErrorInvalidValue, "tiled GEMM: products with x need a k-major A" };
+	else if (a_kmajor) hipLaunchKernelGGL((k_tile_gemm_f64<true, false>), grid, block, 0, s, terms, items, b, x, udot);
+	else hipLaunchKernelGGL((k_tile_gemm_f64<false, false>), grid, block, 0, s, terms, items, b, x, udot);
 	CTG_HIP(hipGetLastError());
 }
 

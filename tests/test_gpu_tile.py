@@ -30,19 +30,53 @@ def dense_problem(da, db, d, D, seed):
     return ts, np.einsum("amx,mqac->xqc", l[0], t2, optimize=True).reshape(-1)
 
 
-@pytest.mark.parametrize("da,db,d,D", [(1, 1, 1, 1), (1, 3, 2, 2), (15, 17, 1, 1), (16, 16, 2, 1), (17, 15, 3, 1), (33, 64, 1, 2), (48, 5, 1, 3),
-                                       (63, 65, 2, 1), (64, 32, 1, 1), (65, 33, 2, 2), (130, 129, 1, 2), (3, 200, 4, 5), (200, 3, 4, 5)])
-def test_tile_form_edges(da, db, d, D, monkeypatch):
+EDGES = [(1, 1, 1, 1), (1, 3, 2, 2), (15, 17, 1, 1), (16, 16, 2, 1), (17, 15, 3, 1), (33, 64, 1, 2), (48, 5, 1, 3),
+                                 (63, 65, 2, 1), (64, 32, 1, 1), (65, 33, 2, 2), (130, 129, 1, 2), (3, 200, 4, 5), (200, 3, 4, 5)]
+
+
+@pytest.mark.parametrize("stage3", ["tasks", "split"])
+@pytest.mark.parametrize("da,db,d,D", EDGES)
+def test_tile_form_edges(da, db, d, D, stage3, monkeypatch):
     monkeypatch.setenv("CT_GEMM_LDS", "1")
     monkeypatch.setenv("CT_STAGE12", "separate")
+    monkeypatch.setenv("CT_STAGE3", stage3)
     ts, want = dense_problem(da, db, d, D, 100 * da + db)
     plan = ct.MatvecPlan(*ts, ct.GROUPED_FP64)
     forms = plan.forms()[0]
     print("case", da, db, d, D, "forms", forms, flush=True)
     sys.stdout.flush()
-    assert forms[0] == 6 and forms[2] == 6
+    assert forms[0] == 6 and forms[2] == (7 if stage3 == "split" else 6)
     x, y = ct.DeviceArray.from_numpy(ts[0].serialize()), ct.DeviceArray(plan.dim)
     plan.apply(x, y)
     plan.synchronize()
     # three chained FP64 products of at most 1000 terms: 2e-16 sqrt(1000) each way
     assert np.linalg.norm(y.numpy() - want) <= 2e-14 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("model,L,chi", [("hubbard", 8, 24), ("xxz", 32, 256), ("hubbard", 32, 256)])
+def test_split_stage3_and_its_lanczos(model, L, chi, monkeypatch):
+    """The k range of every y block cut into slots (CT_STAGE3=split) against the tasks: the matvec, and the
+    Lanczos recurrence whose step adds the slots and takes alpha from the tiles' partials."""
+    monkeypatch.setenv("CT_STAGE12", "separate")
+    p = ct.generate_matvec_problem(model, L, chi, 11)
+    got = {}
+    for stage3 in ("tasks", "split"):
+        monkeypatch.setenv("CT_STAGE3", stage3)
+        plan = ct.MatvecPlan(*p, ct.GROUPED_FP64)
+        assert (plan.forms()[0][2] == 7) == (stage3 == "split")
+        x, y = ct.DeviceArray.from_numpy(p[0].serialize()), ct.DeviceArray(plan.dim)
+        plan.apply(x, y)
+        plan.synchronize()
+        first = plan.lanczos(x, 12)
+        again = plan.lanczos(x, 12)           # the captured recurrence, replayed
+        assert first[0] == again[0] and np.array_equal(first[1].numpy(), again[1].numpy())
+        monkeypatch.setenv("CT_LANCZOS_GRAPH", "0")
+        eager = plan.lanczos(x, 12)
+        monkeypatch.delenv("CT_LANCZOS_GRAPH")
+        assert eager[0] == first[0] and np.array_equal(eager[1].numpy(), first[1].numpy())
+        got[stage3] = (y.numpy(), first[0], first[1].numpy())
+    a, b = got["tasks"], got["split"]
+    assert np.linalg.norm(a[0] - b[0]) <= 1e-14 * np.linalg.norm(a[0])
+    # twelve steps of the recurrence, each carrying rounding of 1e-15 into the next
+    assert abs(a[1] - b[1]) <= 1e-12 * abs(a[1])
+    assert np.linalg.norm(a[2] - b[2]) <= 1e-10
