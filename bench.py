@@ -421,7 +421,7 @@ def main():
         traffic_source = "--hbm-traffic-kib"
     y_g = forms["grouped_fp64"]["y"].numpy()
     names = ["k_grouped_gemm_f64", "k_stream_gemm_f64_wave", "k_grouped_gemm_f64_wg", "k_stream_gemm_f64_wg", "k_wapply", "k_f12",
-             "k_tile_gemm_f64", "k_tile_gemm_f64"]
+             "k_tile_gemm_f64", "k_tile_gemm_f64", "k_wtile"]
     if head == "fused_fp64":
         kernel_name = "k_fused_matvec"
     elif head == "pair_fp64":

@@ -15,7 +15,7 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libchemtensor_gpu.so")
 
-HIP_SOURCES = ["kernels.hip", "tile.hip", "fused.hip", "pair.hip", "runtime.hip", "engine.hip", "lanczos.hip", "split.hip", "dmrg.hip", "serve.hip", "capi.hip"]
+HIP_SOURCES = ["kernels.hip", "tile.hip", "wtile.hip", "fused.hip", "pair.hip", "runtime.hip", "engine.hip", "lanczos.hip", "split.hip", "dmrg.hip", "serve.hip", "capi.hip"]
 CPP_SOURCES = ["host_tensor.cpp", "host_linalg.cpp", "host_models.cpp", "host_molecular.cpp", "host_bond.cpp", "host_io.cpp"]
 # save_mps / load_mps use the HDF5 C library through libchemtensor_h5.so, built only where HDF5's
 # header and library are found (HDF5_ROOT, else the prefixes below)

@@ -329,8 +329,13 @@ struct F12Item { WaUnit u; int g0, ng, a0, ta, c0, tc, lds, pad; };
 constexpr int F12_LDS = 1024;    // doubles of LDS staging per wavefront (8 KB: 20 wavefronts per CU)
 constexpr int F12_RMAX = 16;     // largest number of W_D rows
 
+// the (M,Q) and (P,N) blocks of a class, in row and column order
+struct WaClass { int R = 0, K = 0; std::vector<std::pair<ct_long, ct_long>> rows, cols; };
+
 struct WApplyHost
 {
+	std::vector<WaClass> classes;
+	std::vector<int> unit_class;
 	std::vector<WaUnit> units;
 	std::vector<WaItem> items;
 	std::vector<F12Group> groups;
@@ -359,10 +364,37 @@ struct WApply
 	int nitems = 0;
 	int kmax = 0;
 	bool ok = false;                     // every class fits WA_KMAX columns
-	void upload(const WApplyHost& h, const double* w, hipStream_t s);
+	// offsets: also the offset tables when the column stream does not apply (for the row tiles)
+	void upload(const WApplyHost& h, const double* w, hipStream_t s, bool offsets = false);
 	void release();
 };
 void launch_wapply(const WApply& wa, const double* t1, double* t2, hipStream_t s);
+
+// Stage 2 of classes beyond WA_KMAX columns (wtile.hip): 64-row tiles of W_D that keep only the columns some
+// row of them uses. The entries of W that are zero are left out like blocks that are absent.
+struct WtTile { int np, klist, rlist, mask; int64_t pack; int cost; };   // panels, lists / masks / pack indices
+struct WtItem { int64_t kb, rb, t1_off, t2_off, pack; int t1_bytes, t2_bytes, dA, dC, j0, np, klist, rlist, mask, pad; };
+struct WtHost
+{
+	std::vector<WtItem> items;
+	std::vector<int> lists;        // per tile: 64 rows of the class, then its columns (-1: none)
+	std::vector<uint32_t> masks;   // per panel: bit 4 step + sub-tile
+	std::vector<double> pack;      // per panel: 16 columns x 64 rows in fragment order
+};
+struct WTiles
+{
+	WtItem* items = nullptr;
+	int* lists = nullptr;
+	uint32_t* masks = nullptr;
+	double* pack = nullptr;
+	int nitems = 0;
+	bool ok = false, use = false;
+	void upload(const WtHost& h, hipStream_t s);
+	void release();
+};
+// w: W's entries on the host; false when a class has too many columns or a block pair spans 1 GiB
+bool plan_wtiles(WtHost& h, const WApplyHost& wa, const Meta& W, const double* w);
+void launch_wtiles(const WTiles& wt, const WApply& wa, const double* t1, double* t2, hipStream_t s);
 // stages 1 and 2 fused: T2 from theta (x) and R directly
 void launch_f12(const WApply& wa, const double* x, const double* r, double* t2, hipStream_t s);
 
@@ -562,6 +594,7 @@ struct MatvecPlan
 	bool use_wapply = false;
 	bool use_f12 = false;                       // stages 1 and 2 fused (no T1 in HBM)
 	Stage3Split split3;
+	WTiles wtiles;                              // stage 2 of classes beyond the column stream
 	// fused form: one launch
 	FusedPlan fused;
 	// sector-pair form: one unit launch and one reduction launch
@@ -606,11 +639,11 @@ void merge_grouped_tables(GroupedTables& dst, const GroupedTables& src, int64_t 
 void validate_matvec_operands(const Meta& theta, const Meta& w, const Meta& l, const Meta& r);
 // time every launch form of each grouped stage (and the column-stream stage 2 when available) and
 // keep the fastest; sets *use_wapply
-void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, bool* use_wapply, bool* use_f12, Stage3Split* split3, int64_t nx,
-	hipStream_t s, float (*tuned_ms)[GEMM_NUM_FORMS]);
+void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, bool* use_wapply, bool* use_f12, WTiles* wt, Stage3Split* split3,
+	int64_t nx, hipStream_t s, float (*tuned_ms)[GEMM_NUM_FORMS]);
 // one grouped matvec: stage 1, stage 2 (MFMA tiles or column stream), stage 3
-void launch_grouped_stages(const DevGemm* stage, const GemmBases* bases, const WApply* wa, bool use_wapply, bool use_f12, const Stage3Split* split3,
-	const double* x, double* y, hipStream_t s, hipEvent_t* ev);
+void launch_grouped_stages(const DevGemm* stage, const GemmBases* bases, const WApply* wa, bool use_wapply, bool use_f12, const WTiles* wt,
+	const Stage3Split* split3, const double* x, double* y, hipStream_t s, hipEvent_t* ev);
 
 // stages 1 and 2 and the tiles of the split stage 3 with the alpha partials <y, x> (split3.sum.nunits)
 void launch_grouped_units(const MatvecPlan& p, const double* x, double* udot);

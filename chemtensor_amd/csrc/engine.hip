@@ -656,6 +656,7 @@ MatvecPlan::~MatvecPlan()
 {
 	for (int i = 0; i < 3; i++) stage[i].release();
 	split3.release();
+	wtiles.release();
 	wapply.release();
 	fused.release();
 	pair.release();
@@ -786,7 +787,7 @@ void plan_grouped_tables(GroupedTables& g, const Meta& th, const Meta& W, const 
 	// column-stream form of stage 2: classes D = qM + qQ = qP + qN, one unit per block pair (A,C)
 	{
 		WApplyHost& wa = g.wa;
-		struct Cls { int64_t wrow = 0, wcol = 0; int K = 0, R = 0; std::vector<std::pair<ct_long, ct_long>> rows, cols; };
+		struct Cls { int64_t wrow = 0, wcol = 0; int K = 0, R = 0, id = 0; std::vector<std::pair<ct_long, ct_long>> rows, cols; };
 		std::map<qnumber, Cls> classes;
 		auto get_class = [&](qnumber D) -> const Cls& {
 			auto it = classes.find(D);
@@ -822,6 +823,8 @@ void plan_grouped_tables(GroupedTables& g, const Meta& th, const Meta& W, const 
 					for (int k = 0; k < WA_KMAX; k++) colT[(size_t)k * F12_RMAX + r] = wa.widx[(size_t)(c.wrow + r) * WA_KMAX + k];
 				wa.widxT.insert(wa.widxT.end(), colT.begin(), colT.end());
 			}
+			c.id = (int)wa.classes.size();
+			wa.classes.push_back(WaClass{ c.R, c.K, c.rows, c.cols });
 			return classes.emplace(D, std::move(c)).first->second;
 		};
 		for (ct_long A = 0; A < nA; A++) for (ct_long C = 0; C < nC; C++) {
@@ -858,6 +861,7 @@ void plan_grouped_tables(GroupedTables& g, const Meta& th, const Meta& W, const 
 			}
 			const int unit = (int)wa.units.size();
 			wa.units.push_back(u);
+			wa.unit_class.push_back(c.id);
 			for (int col0 = 0; col0 < (int)(dA * dC); col0 += 64) wa.items.push_back(WaItem{ u, unit, col0 });
 			// fused stages 1 + 2: one group per column group (P,N) of the class
 			if (lean) { wa.f12_ok = false; continue; }
@@ -1051,6 +1055,44 @@ int check_grouped_tables(const Meta& th, const Meta& W, const Meta& L, const Met
 		if (k0 != k1 || !once(wr)) return 9;
 	}
 	const WApplyHost& wa = g.wa;
+	if (wa.kmax > WA_KMAX) {
+		// the row tiles of an operator with one entry in five: every T2 entry written once, every non-zero
+		// entry of W in one pack, and in a sub-tile that its panel's mask runs
+		std::vector<double> wv((size_t)W.nelem, 0.0);
+		size_t nnz = 0, packed = 0;
+		for (size_t i = 0; i < wv.size(); i++) if (i * 2654435761u % 5 == 0) wv[i] = 1.0 + (double)i;
+		WtHost h;
+		if (plan_wtiles(h, wa, W, wv.data())) {
+			for (double v : wv) nnz += v != 0.0;
+			for (size_t i = 0; i < h.pack.size(); i++) {
+				if (h.pack[i] == 0.0) continue;
+				packed++;
+				const size_t p = i / 1024, o = i % 1024, st = o / 256, sub = o / 128 % 2 * 2 + o % 2;
+				if (!(h.masks[p] >> (4 * st + sub) & 1)) return 10;
+			}
+			// entries of W outside every class act on no block
+			if (packed > nnz) return 10;
+			std::vector<int> ws((size_t)g.t2_elems, 0);
+			for (const WtItem& it : h.items) {
+				const int dCp = (it.dC + 1) & ~1;
+				if (it.np < 1 || it.np * 16 > 2048 || (size_t)(it.klist + 16 * it.np) > h.lists.size() || (size_t)(it.mask + it.np) > h.masks.size() ||
+					(size_t)it.pack + (size_t)it.np * 1024 > h.pack.size() || it.t1_off + it.t1_bytes / 8 > g.t1_elems || it.t2_off + it.t2_bytes / 8 > g.t2_elems) return 10;
+				for (int i = 0; i < 64; i++) {
+					const int r = h.lists[(size_t)(it.rlist + i)];
+					const int64_t b = r >= 0 ? wa.rbase[(size_t)(it.rb + r)] : -1;
+					if (b < 0) continue;
+					for (int j = it.j0; j < it.j0 + 64; j++) {
+						const int a = j / dCp, c = j - a * dCp;
+						if (a >= it.dA || c >= it.dC) continue;
+						const int64_t e = b + (int64_t)a * wa.rstride[(size_t)(it.rb + r)] + c;
+						if (e < it.t2_off || e >= it.t2_off + it.t2_bytes / 8) return 10;
+						ws[(size_t)e]++;
+					}
+				}
+			}
+			if (!once(ws)) return 10;
+		}
+	}
 	if (wa.kmax <= WA_KMAX) {
 		std::vector<int> ws((size_t)g.t2_elems, 0);
 		for (const WaItem& it : wa.items) {
@@ -1129,7 +1171,14 @@ static void build_grouped(MatvecPlan& p, bool lean)
 	p.stage_bases[2] = GemmBases{ p.l.d, p.interm[1].d, nullptr };
 	// the column-stream stage 2 (FP64 FMAs, no MFMA) serves the FP64 and the split-FP32 forms: in
 	// both the MFMA GEMMs are stages 1 and 3
-	if (p.mode == CT_MATVEC_GROUPED_FP64 || p.mode == CT_MATVEC_GROUPED_SPLIT) p.wapply.upload(g.wa, p.w.d, p.stream);
+	const bool wide = tiles && g.wa.kmax > WA_KMAX;
+	if (p.mode == CT_MATVEC_GROUPED_FP64 || p.mode == CT_MATVEC_GROUPED_SPLIT) p.wapply.upload(g.wa, p.w.d, p.stream, wide);
+	if (wide) {
+		// the row tiles are made from the entries of W that are not zero
+		const HostPacked w = download_packed(p.w, p.stream);
+		WtHost h;
+		if (plan_wtiles(h, g.wa, p.w.meta, w.v.data())) p.wtiles.upload(h, p.stream);
+	}
 	p.nterms = g.s1.terms.size() + g.s2.terms.size() + g.s3.terms.size();
 	p.ntasks = g.s1.tasks.size() + g.s2.tasks.size() + g.s3.tasks.size();
 	p.nitems = p.stage[0].nitems + p.stage[1].nitems + p.stage[2].nitems;
@@ -1230,7 +1279,8 @@ static void build_plain(MatvecPlan& p)
 // warm-up and three timed launches, HIP events on the plan stream); the fastest form is kept.
 // time every launch form of each grouped stage on the plan's own descriptors (x = 1, y scratch)
 // and keep the fastest; stage 2 also tries the column-stream form
-void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, bool* use_wapply, bool* use_f12, Stage3Split* split3, int64_t nx, hipStream_t s,
+void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, bool* use_wapply, bool* use_f12, WTiles* wt, Stage3Split* split3,
+	int64_t nx, hipStream_t s,
 	float (*tuned_ms)[GEMM_NUM_FORMS])
 {
 	double* x = (double*)dev_alloc((size_t)std::max<int64_t>(nx, 1) * sizeof(double));
@@ -1304,6 +1354,15 @@ void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, 
 			if (force && strcmp(force, "stream") == 0) *use_wapply = true;
 		}
 	}
+	if (wt && wt->ok) {
+		const float ms = time3([&] { launch_wtiles(*wt, *wa, bases[1].B, bases[1].C, s); });
+		wt->use = ms < best2;
+		if (wt->use) best2 = ms;
+		// CT_STAGE2=mfma|rowtiles overrides the timing-based choice
+		const char* force = getenv("CT_STAGE2");
+		if (force && strcmp(force, "mfma") == 0) wt->use = false;
+		if (force && strcmp(force, "rowtiles") == 0) wt->use = true;
+	}
 	if (use_f12) {
 		*use_f12 = false;
 		if (wa && wa->ok && wa->f12_ok) {
@@ -1323,8 +1382,8 @@ void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, 
 }
 
 // launch stages 1 and 2 of a grouped matvec
-static void launch_stages12(const DevGemm* stage, const GemmBases* bases, const WApply* wa, bool use_wapply, bool use_f12, const double* x, hipStream_t s,
-	hipEvent_t* ev)
+static void launch_stages12(const DevGemm* stage, const GemmBases* bases, const WApply* wa, bool use_wapply, bool use_f12, const WTiles* wt, const double* x,
+	hipStream_t s, hipEvent_t* ev)
 {
 	const bool f12 = use_f12 && wa && wa->f12_ok;
 	for (int st = 0; st < 2; st++) {
@@ -1333,6 +1392,7 @@ static void launch_stages12(const DevGemm* stage, const GemmBases* bases, const 
 		if (st == 0 && f12) launch_f12(*wa, x, b.B, bases[1].C, s);
 		else if (st == 1 && f12) { /* done by the fused launch */ }
 		else if (st == 1 && use_wapply && wa && wa->ok) launch_wapply(*wa, b.B, b.C, s);
+		else if (st == 1 && wt && wt->use) launch_wtiles(*wt, *wa, b.B, b.C, s);
 		else launch_grouped_gemm_f64(stage[st], b, s);
 		if (ev) CTG_HIP(hipEventRecord(ev[st + 1], s));
 	}
@@ -1340,14 +1400,14 @@ static void launch_stages12(const DevGemm* stage, const GemmBases* bases, const 
 
 void launch_grouped_units(const MatvecPlan& p, const double* x, double* udot)
 {
-	launch_stages12(p.stage, p.stage_bases, &p.wapply, p.use_wapply, p.use_f12, x, p.stream, nullptr);
+	launch_stages12(p.stage, p.stage_bases, &p.wapply, p.use_wapply, p.use_f12, &p.wtiles, x, p.stream, nullptr);
 	launch_stage3_units(p.split3, p.stage_bases[2], p.stream, x, udot);
 }
 
-void launch_grouped_stages(const DevGemm* stage, const GemmBases* bases, const WApply* wa, bool use_wapply, bool use_f12, const Stage3Split* split3,
-	const double* x, double* y, hipStream_t s, hipEvent_t* ev)
+void launch_grouped_stages(const DevGemm* stage, const GemmBases* bases, const WApply* wa, bool use_wapply, bool use_f12, const WTiles* wt,
+	const Stage3Split* split3, const double* x, double* y, hipStream_t s, hipEvent_t* ev)
 {
-	launch_stages12(stage, bases, wa, use_wapply, use_f12, x, s, ev);
+	launch_stages12(stage, bases, wa, use_wapply, use_f12, wt, x, s, ev);
 	GemmBases b = bases[2];
 	b.C = y;
 	if (split3 && split3->use) {
@@ -1360,7 +1420,7 @@ void launch_grouped_stages(const DevGemm* stage, const GemmBases* bases, const W
 
 static void autotune_stages(MatvecPlan& p)
 {
-	autotune_grouped(p.stage, p.stage_bases, &p.wapply, &p.use_wapply, &p.use_f12, &p.split3, p.theta_meta.nelem, p.stream, p.tuned_ms);
+	autotune_grouped(p.stage, p.stage_bases, &p.wapply, &p.use_wapply, &p.use_f12, &p.wtiles, &p.split3, p.theta_meta.nelem, p.stream, p.tuned_ms);
 	if (p.use_f12 && p.wapply.f12_ok) {
 		// one launch for stages 1 and 2: theta, R and W in, T2 out (T1 never written)
 		const double t1 = (double)p.interm[0].meta.nelem;
@@ -1513,6 +1573,7 @@ float matvec_stage_time(MatvecPlan& p, int stage, const double* x, double* y, in
 		}
 		else if (stage < 2 && p.use_f12 && p.wapply.f12_ok) { if (stage == 0) launch_f12(p.wapply, x, b.B, p.stage_bases[1].C, s); }
 		else if (stage == 1 && p.use_wapply && p.wapply.ok) launch_wapply(p.wapply, b.B, b.C, s);
+		else if (stage == 1 && p.wtiles.use) launch_wtiles(p.wtiles, p.wapply, b.B, b.C, s);
 		else if (stage == 2 && p.split3.use) {
 			launch_stage3_units(p.split3, b, s);
 			launch_pair_reduce(p.split3.sum, y, s);
@@ -1560,7 +1621,7 @@ void matvec_apply(MatvecPlan& p, const double* x, double* y, float* stage_ms)
 			if (stage_ms) CTG_HIP(hipEventRecord(p.ev[st + 1], s));
 		}
 	}
-	else launch_grouped_stages(p.stage, p.stage_bases, &p.wapply, p.use_wapply, p.use_f12, &p.split3, x, y, s, stage_ms ? p.ev : nullptr);
+	else launch_grouped_stages(p.stage, p.stage_bases, &p.wapply, p.use_wapply, p.use_f12, &p.wtiles, &p.split3, x, y, s, stage_ms ? p.ev : nullptr);
 	if (stage_ms) {
 		CTG_HIP(hipEventSynchronize(p.ev[3]));
 		for (int st = 0; st < 3; st++) CTG_HIP(hipEventElapsedTime(&stage_ms[st], p.ev[st], p.ev[st + 1]));

@@ -1052,17 +1052,18 @@ static T* upload_array(const std::vector<T>& v, hipStream_t s)
 	return d;
 }
 
-void WApply::upload(const WApplyHost& h, const double* w, hipStream_t s)
+void WApply::upload(const WApplyHost& h, const double* w, hipStream_t s, bool offsets)
 {
 	release();
 	ok = h.kmax <= WA_KMAX;
-	if (!ok) return;
-	units = upload_array(h.units, s);
-	items = upload_array(h.items, s);
+	if (!ok && !offsets) return;
 	kbase = upload_array(h.kbase, s);
 	rbase = upload_array(h.rbase, s);
 	kstride = upload_array(h.kstride, s);
 	rstride = upload_array(h.rstride, s);
+	if (!ok) return;
+	units = upload_array(h.units, s);
+	items = upload_array(h.items, s);
 	int64_t* widx = upload_array(h.widx, s);
 	const int64_t n = (int64_t)h.widx.size();
 	wmat = (double*)dev_alloc((size_t)std::max<int64_t>(n, 1) * sizeof(double));

@@ -11,8 +11,9 @@ import chemtensor_amd as ct
 pytestmark = pytest.mark.gpu
 
 
-def dense_problem(da, db, d, D, seed):
-    """One sector on every axis: stage 1 is a (da d) x (D db) product with K = db, stage 3 da x (d db) with K = da D."""
+def dense_problem(da, db, d, D, seed, density=1.0):
+    """One sector on every axis: stage 1 is a (da d) x (D db) product with K = db, stage 3 da x (d db) with K = da D;
+    a share `density` of the operator's entries is not zero."""
     rng = np.random.default_rng(seed)
     z = lambda n: np.zeros(n, dtype=np.int32)
     shapes = [(da, d, db), (D, d, d, D), (1, da, D, da), (db, D, db, 1)]
@@ -21,6 +22,8 @@ def dense_problem(da, db, d, D, seed):
     for s, ad in zip(shapes, dirs):
         t = ct.HostTensor.zeros(s, ad, [z(n) for n in s])
         v = rng.standard_normal(s)
+        if len(ts) == 1 and density < 1:
+            v *= rng.random(s) < density
         t.deserialize(v.reshape(-1))
         ts.append(t)
         vs.append(v)
@@ -80,3 +83,19 @@ def test_split_stage3_and_its_lanczos(model, L, chi, monkeypatch):
     # twelve steps of the recurrence, each carrying rounding of 1e-15 into the next
     assert abs(a[1] - b[1]) <= 1e-12 * abs(a[1])
     assert np.linalg.norm(a[2] - b[2]) <= 1e-10
+
+
+@pytest.mark.parametrize("density", [0.0, 0.02, 0.3, 1.0])
+@pytest.mark.parametrize("da,db,d,D", [(1, 1, 2, 20), (3, 5, 4, 17), (17, 9, 2, 33), (5, 64, 3, 48), (33, 2, 2, 65), (1, 129, 1, 40)])
+def test_row_tiles_of_wide_classes(da, db, d, D, density, monkeypatch):
+    """Stage 2 as row tiles that keep the columns in use (CT_STAGE2=rowtiles): rows beyond a multiple of 64,
+    columns beyond a multiple of 16, odd column counts, empty and full operators."""
+    monkeypatch.setenv("CT_STAGE2", "rowtiles")
+    ts, want = dense_problem(da, db, d, D, 7 * da + db, density)
+    plan = ct.MatvecPlan(*ts, ct.GROUPED_FP64)
+    print("case", da, db, d, D, density, "forms", plan.forms()[0], flush=True)
+    assert plan.forms()[0][1] == 8
+    x, y = ct.DeviceArray.from_numpy(ts[0].serialize()), ct.DeviceArray(plan.dim)
+    plan.apply(x, y)
+    plan.synchronize()
+    assert np.linalg.norm(y.numpy() - want) <= 2e-14 * np.linalg.norm(want)
