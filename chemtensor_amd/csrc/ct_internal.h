@@ -576,9 +576,13 @@ bool split_stage3(const GemmBatch& s3, int panels, GemmBatch& out, std::vector<P
 // y partial blocks of stage 3, with the alpha partials <y, x> per tile when udot is given
 void launch_stage3_units(const Stage3Split& sp, GemmBases b, hipStream_t s, const double* x = nullptr, double* udot = nullptr);
 
-// a Lanczos step on the split stage 3 has one launch less than on the tasks (the step adds the slots, the
-// tiles write the alpha partials): worth this much (ms)
+// A Lanczos step on the split stage 3 has one launch less than on the tasks (the step adds the slots, the
+// tiles write the alpha partials): worth this much (ms). Taken from vectors of LZ_SPLIT_MIN entries on (20 steps
+// on sweep-like bonds, tasks against split: XXZ 250 states, 63000 entries, 739 against 641 us, 500 states 1202
+// against 1096, Hubbard 500 states 1044 against 991; below, at 2000 to 15000 entries, 427 against 418 and 478
+// against 472, hardly more than two runs differ by).
 constexpr float LZ_SAVED_MS = 0.006f;
+constexpr int64_t LZ_SPLIT_MIN = (int64_t)1 << 15;
 
 struct MatvecPlan
 {
@@ -691,7 +695,6 @@ struct BatchPlan
 	WApply wapply;
 	bool use_wapply = false;
 	bool use_f12 = false;
-	Stage3Split split3;
 	double* t1 = nullptr;
 	double* t2 = nullptr;
 	bool use_fused = false;                     // the faster of the two forms, timed at plan creation

@@ -525,7 +525,6 @@ BatchPlan::~BatchPlan()
 {
 	fused.release();
 	for (int i = 0; i < 3; i++) stage[i].release();
-	split3.release();
 	wapply.release();
 	dev_free(t1);
 	dev_free(t2);
@@ -609,13 +608,12 @@ BatchPlan* build_batch_plan(std::vector<BatchInput>& in, hipStream_t s, bool tun
 	b->stage[0].upload(g.s1, s, tune);
 	b->stage[1].upload(g.s2, s, tune);
 	b->stage[2].upload(g.s3, s, tune);
-	if (tune) b->split3.build(g.s3, s);
 	b->stage_bases[0] = GemmBases{ nullptr, b->r, b->t1 };
 	b->stage_bases[1] = GemmBases{ b->w, b->t1, b->t2 };
 	b->stage_bases[2] = GemmBases{ b->l, b->t2, nullptr };
 	b->wapply.upload(g.wa, b->w, s);
 	if (tune) {
-		autotune_grouped(b->stage, b->stage_bases, &b->wapply, &b->use_wapply, &b->use_f12, nullptr, &b->split3, nx, s, nullptr);
+		autotune_grouped(b->stage, b->stage_bases, &b->wapply, &b->use_wapply, &b->use_f12, nullptr, nullptr, nx, s, nullptr);
 		b->fused_ok = build_fused_batch(b->fused, probs, s);
 	}
 	else {
@@ -699,7 +697,7 @@ void batch_apply(BatchPlan& b, const double* x, double* y)
 		launch_fused_matvec(b.fused, x, b.w, b.l, b.r, y, b.stream);
 		return;
 	}
-	launch_grouped_stages(b.stage, b.stage_bases, &b.wapply, b.use_wapply, b.use_f12, nullptr, &b.split3, x, y, b.stream, nullptr);
+	launch_grouped_stages(b.stage, b.stage_bases, &b.wapply, b.use_wapply, b.use_f12, nullptr, nullptr, x, y, b.stream, nullptr);
 }
 
 }  // namespace ctg

@@ -247,7 +247,14 @@ __global__ __launch_bounds__(LZ_THREADS) void k_lz_ritz(const double* __restrict
 	for (int64_t i = (int64_t)blockIdx.x * LZ_THREADS + threadIdx.x; i < n; i += (int64_t)gridDim.x * LZ_THREADS) {
 		for (int k = 0; k < numeig; k++) {
 			double acc = 0;
-			for (int j = 0; j < numiter; j++) acc += V[(int64_t)j * n + i] * z[j * numeig + k];
+			for (int j0 = 0; j0 < numiter; j0 += 8) {
+				double v[8];
+				#pragma unroll
+				for (int q = 0; q < 8; q++) v[q] = V[(int64_t)min(j0 + q, numiter - 1) * n + i];
+				#pragma unroll
+				for (int q = 0; q < 8; q++)
+					if (j0 + q < numiter) acc += v[q] * z[(j0 + q) * numeig + k];
+			}
 			u[i * numeig + k] = acc;
 		}
 	}
@@ -511,6 +518,12 @@ __device__ __forceinline__ double sum_range(const double* __restrict__ part, int
 	return block_sum(v, sh);
 }
 
+// A segment has up to 16 entries per thread (more in vectors beyond 2^18), which a thread takes in the same
+// order as before but loads eight at a time: with some sixty segments on the chip the kernels below are bound
+// by the latency of their loads (16 problems of up to 256 states, per step: dot 7.0, alpha update 10.6, beta
+// scale 5.5 us with one load at a time; Ritz vectors 81 us).
+constexpr int BLZ_PRE = 8;
+
 __global__ __launch_bounds__(LZ_THREADS) void k_blz_dot_partial(const double* __restrict__ x, const double* __restrict__ y, const LzSeg* __restrict__ segs,
 	double* __restrict__ part, const double* __restrict__ scal, int S, int check_stop)
 {
@@ -518,7 +531,18 @@ __global__ __launch_bounds__(LZ_THREADS) void k_blz_dot_partial(const double* __
 	const LzSeg g = segs[blockIdx.x];
 	if (check_stop && scal[g.prob * S + S - 1] != 0) return;
 	double v = 0;
-	for (int64_t i = g.begin + threadIdx.x; i < g.end; i += LZ_THREADS) v += x[i] * y[i];
+	for (int64_t i0 = g.begin + threadIdx.x; i0 < g.end; i0 += BLZ_PRE * LZ_THREADS) {
+		double a[BLZ_PRE], b[BLZ_PRE];
+		#pragma unroll
+		for (int k = 0; k < BLZ_PRE; k++) {
+			const int64_t i = min(i0 + k * LZ_THREADS, g.end - 1);
+			a[k] = x[i];
+			b[k] = y[i];
+		}
+		#pragma unroll
+		for (int k = 0; k < BLZ_PRE; k++)
+			if (i0 + k * LZ_THREADS < g.end) v += a[k] * b[k];
+	}
 	const double s = block_sum(v, sh);
 	if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
@@ -543,17 +567,37 @@ __global__ __launch_bounds__(LZ_THREADS) void k_blz_alpha_update(double* __restr
 	double* sc = scal + (int64_t)g.prob * S;
 	if (sc[S - 1] != 0) return;
 	const LzProb q = probs[g.prob];
+	double wv[BLZ_PRE], a[BLZ_PRE], b[BLZ_PRE];
+	auto load = [&](int64_t i0) {
+		if (g.end <= g.begin) return;   // a problem without entries
+		#pragma unroll
+		for (int k = 0; k < BLZ_PRE; k++) {
+			const int64_t i = min(i0 + k * LZ_THREADS, g.end - 1);
+			wv[k] = w[i];
+			a[k] = vj[i];
+			b[k] = j > 0 ? vjm1[i] : 0.0;
+		}
+	};
+	// the first entries' loads cover the sum of the partials
+	if (j < maxiter - 1) load(g.begin + threadIdx.x);
 	const double alpha = sum_range(part, q.b0, q.b1, sh);
 	if ((int)blockIdx.x == q.b0 && threadIdx.x == 0) sc[j] = alpha;
 	if (j == maxiter - 1) return;
 	const double bprev = (j > 0) ? sc[maxiter + j - 1] : 0.0;
 	double v = 0;
-	for (int64_t i = g.begin + threadIdx.x; i < g.end; i += LZ_THREADS) {
-		double wi = w[i];
-		if (j > 0) wi -= alpha * vj[i] + bprev * vjm1[i];
-		else wi -= alpha * vj[i];
-		w[i] = wi;
-		v += wi * wi;
+	for (int64_t i0 = g.begin + threadIdx.x; i0 < g.end; i0 += BLZ_PRE * LZ_THREADS) {
+		if (i0 != g.begin + threadIdx.x) load(i0);
+		#pragma unroll
+		for (int k = 0; k < BLZ_PRE; k++) {
+			const int64_t i = i0 + k * LZ_THREADS;
+			if (i < g.end) {
+				double wi = wv[k];
+				if (j > 0) wi -= alpha * a[k] + bprev * b[k];
+				else wi -= alpha * a[k];
+				w[i] = wi;
+				v += wi * wi;
+			}
+		}
 	}
 	const double s = block_sum(v, sh);
 	if (threadIdx.x == 0) part2[blockIdx.x] = s;
@@ -568,6 +612,13 @@ __global__ __launch_bounds__(LZ_THREADS) void k_blz_beta_scale(const double* __r
 	double* sc = scal + (int64_t)g.prob * S;
 	if (sc[S - 1] != 0) return;
 	const LzProb q = probs[g.prob];
+	double wv[BLZ_PRE];
+	auto load = [&](int64_t i0) {
+		if (g.end <= g.begin) return;   // a problem without entries
+		#pragma unroll
+		for (int k = 0; k < BLZ_PRE; k++) wv[k] = w[min(i0 + k * LZ_THREADS, g.end - 1)];
+	};
+	load(g.begin + threadIdx.x);
 	const double beta = sqrt(sum_range(part2, q.b0, q.b1, sh));
 	const double thresh = 100.0 * (double)q.n * 2.2204460492503131e-16;   // krylov.c:58
 	if (beta < thresh) {
@@ -577,19 +628,32 @@ __global__ __launch_bounds__(LZ_THREADS) void k_blz_beta_scale(const double* __r
 	}
 	if ((int)blockIdx.x == q.b0 && threadIdx.x == 0) sc[maxiter + j] = beta;
 	const double inv = 1 / beta;
-	for (int64_t i = g.begin + threadIdx.x; i < g.end; i += LZ_THREADS) vnext[i] = inv * w[i];
+	for (int64_t i0 = g.begin + threadIdx.x; i0 < g.end; i0 += BLZ_PRE * LZ_THREADS) {
+		if (i0 != g.begin + threadIdx.x) load(i0);
+		#pragma unroll
+		for (int k = 0; k < BLZ_PRE; k++)
+			if (i0 + k * LZ_THREADS < g.end) vnext[i0 + k * LZ_THREADS] = inv * wv[k];
+	}
 }
 
-// u = sum_{j < numiter_p} z_p[j] V_j on each problem's segment
+// u = sum_{j < numiter_p} z_p[j] V_j on each problem's segment, the BLZ_RITZ blocks of a segment taking turns
+constexpr int BLZ_RITZ = 8;
 __global__ __launch_bounds__(LZ_THREADS) void k_blz_ritz(const double* __restrict__ V, int64_t ntot, const double* __restrict__ z, const int* __restrict__ nit,
 	int maxiter, const LzSeg* __restrict__ segs, double* __restrict__ u)
 {
 	const LzSeg g = segs[blockIdx.x];
 	const int m = nit[g.prob];
 	const double* zp = z + (int64_t)g.prob * maxiter;
-	for (int64_t i = g.begin + threadIdx.x; i < g.end; i += LZ_THREADS) {
+	for (int64_t i = g.begin + (int64_t)blockIdx.y * LZ_THREADS + threadIdx.x; i < g.end; i += BLZ_RITZ * LZ_THREADS) {
 		double acc = 0;
-		for (int jj = 0; jj < m; jj++) acc += V[(int64_t)jj * ntot + i] * zp[jj];
+		for (int j0 = 0; j0 < m; j0 += BLZ_PRE) {
+			double v[BLZ_PRE];
+			#pragma unroll
+			for (int k = 0; k < BLZ_PRE; k++) v[k] = V[(int64_t)min(j0 + k, m - 1) * ntot + i];
+			#pragma unroll
+			for (int k = 0; k < BLZ_PRE; k++)
+				if (j0 + k < m) acc += v[k] * zp[j0 + k];
+		}
 		u[i] = acc;
 	}
 }
@@ -705,7 +769,7 @@ int lanczos_ground_state_batch(BatchPlan& b, const double* vstart, int maxiter, 
 	}
 	CTG_HIP(hipMemcpyAsync(lw.z, zall.data(), zall.size() * sizeof(double), hipMemcpyHostToDevice, s));
 	CTG_HIP(hipMemcpyAsync(lw.nit, nit.data(), nit.size() * sizeof(int), hipMemcpyHostToDevice, s));
-	hipLaunchKernelGGL(k_blz_ritz, dim3(b.nblocks), dim3(LZ_THREADS), 0, s, (const double*)lw.v, ntot, (const double*)lw.z, (const int*)lw.nit, maxiter,
+	hipLaunchKernelGGL(k_blz_ritz, dim3(b.nblocks, BLZ_RITZ), dim3(LZ_THREADS), 0, s, (const double*)lw.v, ntot, (const double*)lw.z, (const int*)lw.nit, maxiter,
 		b.segs, u);
 	CTG_HIP(hipGetLastError());
 	CTG_HIP(hipStreamSynchronize(s));
