@@ -34,7 +34,7 @@ extern "C" {
 void apply_local_hamiltonian(const struct block_sparse_tensor* a, const struct block_sparse_tensor* w, const struct block_sparse_tensor* l, const struct block_sparse_tensor* r, struct block_sparse_tensor* b)
 {
 	try {
-		std::unique_ptr<MatvecPlan> p(build_matvec_plan(a, w, l, r, CT_MATVEC_GROUPED_FP64, false));
+		std::unique_ptr<MatvecPlan> p(build_matvec_plan(a, w, l, r, CT_MATVEC_GROUPED_FP64, false, false));
 		DevTensor x = upload(a, p->stream);
 		// result axes: l axis 3, w axis 1, r axis 2 (chain_ops.c:388); equal to a's axes here
 		DevTensor y(p->theta_meta);

@@ -523,6 +523,7 @@ struct LanczosWork
 	int cap = 0, zcap = 0, pcap = 0;
 	hipGraphExec_t graph = nullptr;    // captured recurrence for 'graph_maxiter' steps
 	int graph_maxiter = 0;
+	int64_t solves = 0;                // ground states computed with it
 	void reserve(int64_t n, int maxiter, int numeig, int partials = 1024);
 	void drop_graph();
 	~LanczosWork();
@@ -675,6 +676,7 @@ struct BatchLanczosWork
 	int cap = 0;
 	hipGraphExec_t graph = nullptr;
 	int graph_maxiter = 0;
+	int64_t solves = 0;
 	void drop_graph();
 	~BatchLanczosWork();
 };
@@ -783,7 +785,8 @@ struct DmrgState
 	size_t device_bytes() const;
 };
 
-MatvecPlan* build_matvec_plan(const block_sparse_tensor* a, const block_sparse_tensor* w, const block_sparse_tensor* l, const block_sparse_tensor* r, int mode, bool autotune);
+MatvecPlan* build_matvec_plan(const block_sparse_tensor* a, const block_sparse_tensor* w, const block_sparse_tensor* l, const block_sparse_tensor* r, int mode, bool autotune,
+	bool reference_count = true);
 MatvecPlan* build_matvec_plan_dev(const Meta& theta, DevTensor&& w, DevTensor&& l, DevTensor&& r, int mode, hipStream_t s, bool autotune,
 	bool reference_count = true);
 void matvec_apply(MatvecPlan& p, const double* x, double* y, float* stage_ms);

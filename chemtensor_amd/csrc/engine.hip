@@ -1538,12 +1538,13 @@ MatvecPlan* build_matvec_plan_dev(const Meta& theta, DevTensor&& w, DevTensor&& 
 	return p;
 }
 
-MatvecPlan* build_matvec_plan(const block_sparse_tensor* a, const block_sparse_tensor* w, const block_sparse_tensor* l, const block_sparse_tensor* r, int mode, bool autotune)
+MatvecPlan* build_matvec_plan(const block_sparse_tensor* a, const block_sparse_tensor* w, const block_sparse_tensor* l, const block_sparse_tensor* r, int mode, bool autotune,
+	bool reference_count)
 {
 	hipStream_t s = default_stream();
 	Meta th = meta_of(a);
 	DevTensor dw = upload(w, s), dl = upload(l, s), dr = upload(r, s);
-	return build_matvec_plan_dev(th, std::move(dw), std::move(dl), std::move(dr), mode, s, autotune);
+	return build_matvec_plan_dev(th, std::move(dw), std::move(dl), std::move(dr), mode, s, autotune, reference_count);
 }
 
 float matvec_stage_time(MatvecPlan& p, int stage, const double* x, double* y, int reps)
