@@ -469,8 +469,11 @@ static bool pair_lz_fused()
 
 int lanczos_ground_state(MatvecPlan& p, const double* vstart, int maxiter, double* lambda, double* u)
 {
-	// the plain form replays thousands of per-block launches; it stays eager
-	const bool graph = p.mode != CT_MATVEC_PLAIN_FP64 && graph_enabled();
+	// the plain form replays thousands of per-block launches; it stays eager. The others capture the recurrence
+	// on a plan's second solve: capture and instantiation of the hundred nodes take longer than they save on
+	// one solve (Hubbard bond of 512 states, first solve of a plan 1.35 to 1.55 ms captured, 1.03 ms eager),
+	// and a sweep makes a plan for each solve
+	const bool graph = p.mode != CT_MATVEC_PLAIN_FP64 && graph_enabled() && p.lz.solves++ > 0;
 	// the sector-pair form computes the alpha partials in its partial-sum launch
 	DevMatvecDot mvd;
 	if (p.mode == CT_MATVEC_PAIR_FP64) {
@@ -701,6 +704,7 @@ int lanczos_ground_state_batch(BatchPlan& b, const double* vstart, int maxiter, 
 {
 	if (maxiter < 1 || b.nprob < 1) return CT_ERR_ARG;
 	BatchLanczosWork& lw = b.lz;
+	use_graph = use_graph && lw.solves++ > 0;   // captured on the second solve, as for a single plan
 	hipStream_t s = b.stream;
 	const int64_t ntot = b.off.back();
 	const int S = 2 * maxiter + 2;
