@@ -110,7 +110,8 @@ def bench_batch(ct, nprob, seed, steps, warmup, lanczos_iter):
     y64, y32 = y.numpy(), ys.numpy()
     split_err = float(np.linalg.norm(y32 - y64) / np.linalg.norm(y64))
     log(f"batch of {nprob} split-FP32: {ms_split:.4f} ms per batched matvec (rel err vs FP64 batch {split_err:.1e}), plan {t_splan:.2f}s")
-    batch.lanczos(x, lanczos_iter)
+    for _ in range(2):                        # the second solve captures the recurrence that later ones replay
+        batch.lanczos(x, lanczos_iter)
     t0 = time.perf_counter()
     reps = 5
     for _ in range(reps):
@@ -237,6 +238,7 @@ def bench_molecular_matvec(ct, n, chi, seed, steps, warmup):
             continue
         y = ct.DeviceArray(plan.dim)
         ms, stage_ms = time_form(ct, plan, x, y, steps, warmup)
+        # rates count every product of the reference; the grouped form leaves those with zeros of W out (about 3/4)
         f = {"ms_per_matvec": round(ms, 5), "tflops": round(plan.flops / (ms * 1e-3) / 1e12, 4),
              "fp64_mfma_peak_frac": round(plan.flops / (ms * 1e-3) / 1e12 / FP64_MFMA_PEAK, 4),
              "stage_ms": [round(float(v), 5) for v in stage_ms]}
@@ -514,7 +516,8 @@ def main():
     v0 = ct.DeviceArray.from_numpy(np.random.default_rng(args.seed).standard_normal(plan.dim))
     for label, flag in (("graph", "1"), ("eager", "0")):
         os.environ["CT_LANCZOS_GRAPH"] = flag
-        plan.lanczos(v0, args.lanczos_iter)
+        for _ in range(2):                    # the second solve captures the recurrence that later ones replay
+            plan.lanczos(v0, args.lanczos_iter)
         t0 = time.perf_counter()
         reps = 20
         for _ in range(reps):
