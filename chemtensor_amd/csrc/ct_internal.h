@@ -501,6 +501,8 @@ void launch_pair_matvec_dot(const PairPlan& pp, const double* x, const double* r
 // summed from the partial blocks, v_j and u_{j+1} written, npart_out[0 .. G) the partials of
 // |u_{j+1}|^2; buffers of pair_step_partials(pp) entries hold either partial set
 int pair_step_partials(const PairPlan& pp);
+// workgroups of that launch for nred reduction items
+int pair_step_grid(int nred);
 void launch_pair_lz_step(const PairPlan& pp, const double* uj, double* unext, double* vj_out, const double* vjm1, int j, int maxiter,
 	const double* dpart, const double* npart, double thresh, double* npart_out, double* scal, hipStream_t s);
 // the same launches with the partial blocks in a file-scope device array of PR_SCRATCH_DOUBLES
@@ -578,12 +580,17 @@ bool split_stage3(const GemmBatch& s3, int panels, GemmBatch& out, std::vector<P
 void launch_stage3_units(const Stage3Split& sp, GemmBases b, hipStream_t s, const double* x = nullptr, double* udot = nullptr);
 
 // A Lanczos step on the split stage 3 has one launch less than on the tasks (the step adds the slots, the
-// tiles write the alpha partials): worth this much (ms). Taken from vectors of LZ_SPLIT_MIN entries on (20 steps
-// on sweep-like bonds, tasks against split: XXZ 250 states, 63000 entries, 739 against 641 us, 500 states 1202
-// against 1096, Hubbard 500 states 1044 against 991; below, at 2000 to 15000 entries, 427 against 418 and 478
-// against 472, hardly more than two runs differ by).
-constexpr float LZ_SAVED_MS = 0.006f;
-constexpr int64_t LZ_SPLIT_MIN = (int64_t)1 << 15;
+// tiles write the alpha partials): worth LZ_SAVED_MS (ms) between vectors of LZ_SPLIT_MIN and of LZ_SPLIT_MAX
+// entries. 20 steps on sweep-like bonds, tasks against split, beside the time that the split takes more or
+// less for one matvec: XXZ 250 states (59000 entries) 716 against 631 us, -1 us; 515 states (272000) 1403
+// against 1219, -6; 1000 states (983000) 3505 against 3414, -4; Hubbard 512 states (245000) 963 against 948,
+// +2; 1000 states (952000) 2128 against 2223, +8. Beyond, a wavefront adds the slots of several items one
+// after another: XXZ 2000 states (3974000) 17800 against 18400, Hubbard 2000 states (3606000) 8020 against
+// 8400. Below, at 2000 to 15000 entries, 427 against 418 and 478 against 472, hardly more than two runs
+// differ by. The two ways round differently at every size: Ritz vectors by 1e-15 on random environments, by
+// 1e-14 on sweep-like ones, with the same sign in 48 pairs of solves of 1 to 20 steps, 240 to 116000 entries.
+constexpr float LZ_SAVED_MS = 0.003f;
+constexpr int64_t LZ_SPLIT_MIN = (int64_t)1 << 15, LZ_SPLIT_MAX = (int64_t)1 << 20;
 
 struct MatvecPlan
 {

@@ -1037,8 +1037,10 @@ int check_grouped_tables(const Meta& th, const Meta& W, const Meta& L, const Met
 			if (!once(cover)) return 8;
 		}
 	// the split stage 3: every partial entry written once from operands in range, every y entry the sum of its
-	// block's slots, every k of a block in one of them
-	for (const int panels : { 1, 6 }) {
+	// block's slots, every k of a block in one of them; the workgroups of a Lanczos step on it, each of which
+	// reads the partials of all tiles and workgroups, read them at most four times as often as the vectors and
+	// partial blocks have entries (2^24 reads, about a microsecond, at any size)
+	for (const int panels : { 1, 6, 24 }) {
 		GemmBatch sp;
 		std::vector<PrRed> red;
 		int64_t elems = 0;
@@ -1053,6 +1055,10 @@ int check_grouped_tables(const Meta& th, const Meta& W, const Meta& L, const Met
 			for (int e = 0; e < r.n; e++) wr[(size_t)(r.y + e)]++;
 		}
 		if (k0 != k1 || !once(wr)) return 9;
+		int64_t tiles = 0;
+		for (const GemmTask& t : sp.tasks) tiles += (int64_t)((t.M + LDS_TILE - 1) / LDS_TILE) * ((t.N + LDS_TILE - 1) / LDS_TILE);
+		const int64_t groups = pair_step_grid((int)red.size());
+		if (panels == 24 && groups * (groups + tiles) > std::max<int64_t>((int64_t)1 << 24, 4 * (th.nelem + elems))) return 11;
 	}
 	const WApplyHost& wa = g.wa;
 	if (wa.kmax > WA_KMAX) {
@@ -1335,7 +1341,7 @@ void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, 
 		if (st == 2 && split3 && split3->ok) {
 			const float ms = time3([&] { launch_stage3_units(*split3, b, s); launch_pair_reduce(split3->sum, y, s); });
 			split3->use = ms < best;
-			split3->use_lanczos = nx >= LZ_SPLIT_MIN && ms - best < LZ_SAVED_MS;
+			split3->use_lanczos = nx >= LZ_SPLIT_MIN && nx <= LZ_SPLIT_MAX && ms - best < LZ_SAVED_MS;
 			// CT_STAGE3=split|tasks overrides the timing-based choice
 			const char* force = getenv("CT_STAGE3");
 			if (force && strcmp(force, "tasks") == 0) split3->use = split3->use_lanczos = false;

@@ -357,6 +357,11 @@ __global__ __launch_bounds__(256) void k_pair_reduce_dot(const PrRed* __restrict
 // same in every workgroup), and per element of one reduction item: y = the sum of its slots in slot
 // order, v_j = u_j / beta, u_{j+1} = y / beta - alpha v_j - beta v_{j-1}, and the partials of
 // |u_{j+1}|^2 per workgroup. The final step (j = maxiter - 1) writes alpha and v_j only.
+// Every workgroup reads all the partials, so at one item per wavefront their traffic would grow with the
+// square of the vector length (Hubbard bond of 2000 states, 3.6e6 entries: 14133 workgroups reading 17352
+// partials each, 2 GB; 20 steps 9870 us, 8400 us with the limit): beyond PR_STEP_GRID workgroups a wavefront
+// takes several items in turn, the first one's loads ahead of the partials.
+constexpr int PR_STEP_GRID = 2048;
 __global__ __launch_bounds__(256) void k_pair_lz_step(const PrRed* __restrict__ items, const int nitems, const double* __restrict__ part,
 	const double* __restrict__ uj, double* __restrict__ unext, double* __restrict__ vj_out, const double* __restrict__ vjm1, int j, int maxiter,
 	const double* __restrict__ dpart, int Gd, const double* __restrict__ npart, int Gn, double thresh, double* __restrict__ npart_out,
@@ -365,11 +370,13 @@ __global__ __launch_bounds__(256) void k_pair_lz_step(const PrRed* __restrict__ 
 	__shared__ double sh[8];
 	if (scal[2 * maxiter + 1] != 0) return;
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-	const int w = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + wave));
+	int w = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + wave));
 	const bool upd = j < maxiter - 1;
 	int64_t i = -1;
 	double yv = 0.0, uv = 0.0, bv = 0.0;
-	if (w < nitems) {
+	auto load = [&]() {
+		i = -1;
+		if (w >= nitems) return;
 		const PrRed it = items[w];
 		if (lane < it.n) {
 			i = it.y + lane;
@@ -379,7 +386,8 @@ __global__ __launch_bounds__(256) void k_pair_lz_step(const PrRed* __restrict__ 
 				if (j > 0) bv = vjm1[i];
 			}
 		}
-	}
+	};
+	load();
 	// beta^2 and <u_j, y>: per-thread strided sums, wavefront butterflies, then the four wavefronts
 	// (thread tid sums entries tid + 256 k in k order, four loads in flight at a time; entries past
 	// the ends add zeros, which leave the sums unchanged)
@@ -428,14 +436,19 @@ __global__ __launch_bounds__(256) void k_pair_lz_step(const PrRed* __restrict__ 
 		if (j > 0) scal[maxiter + j - 1] = beta;
 	}
 	double acc = 0.0;
-	if (i >= 0) {
-		const double v = inv * uv;
-		if (j > 0) vj_out[i] = v;
-		if (upd) {
-			const double wi = (j > 0) ? inv * yv - (alpha * v + beta * bv) : yv - alpha * v;
-			unext[i] = wi;
-			acc = wi * wi;
+	while (true) {
+		if (i >= 0) {
+			const double v = inv * uv;
+			if (j > 0) vj_out[i] = v;
+			if (upd) {
+				const double wi = (j > 0) ? inv * yv - (alpha * v + beta * bv) : yv - alpha * v;
+				unext[i] = wi;
+				acc += wi * wi;
+			}
 		}
+		w += 4 * (int)gridDim.x;
+		if (w >= nitems) break;
+		load();
 	}
 	if (upd) {
 		#pragma unroll
@@ -1336,12 +1349,14 @@ void launch_pair_matvec(const PairPlan& pp, const double* x, const double* r, co
 
 int pair_dot_partials(const PairPlan& pp) { return std::max(1, (pp.nred + 3) / 4); }
 
-int pair_step_partials(const PairPlan& pp) { return std::max(std::max(1, pp.nunits), (pp.nred + 3) / 4); }
+int pair_step_grid(int nred) { return std::max(1, std::min(PR_STEP_GRID, (nred + 3) / 4)); }
+
+int pair_step_partials(const PairPlan& pp) { return std::max(std::max(1, pp.nunits), pair_step_grid(pp.nred)); }
 
 void launch_pair_lz_step(const PairPlan& pp, const double* uj, double* unext, double* vj_out, const double* vjm1, int j, int maxiter,
 	const double* dpart, const double* npart, double thresh, double* npart_out, double* scal, hipStream_t s)
 {
-	const int G = std::max(1, (pp.nred + 3) / 4);
+	const int G = pair_step_grid(pp.nred);
 	hipLaunchKernelGGL(k_pair_lz_step, dim3((unsigned)G), dim3(256), 0, s, (const PrRed*)pp.red, pp.nred, (const double*)pp.part, uj, unext, vj_out, vjm1,
 		j, maxiter, dpart, std::max(0, pp.nunits), npart, G, thresh, npart_out, scal);
 	CTG_HIP(hipGetLastError());

@@ -56,10 +56,11 @@ def test_tile_form_edges(da, db, d, D, stage3, monkeypatch):
     assert np.linalg.norm(y.numpy() - want) <= 2e-14 * np.linalg.norm(want)
 
 
-@pytest.mark.parametrize("model,L,chi", [("hubbard", 8, 24), ("xxz", 32, 256), ("hubbard", 32, 256)])
+@pytest.mark.parametrize("model,L,chi", [("hubbard", 8, 24), ("xxz", 32, 256), ("hubbard", 32, 256), ("xxz", 32, 1200)])
 def test_split_stage3_and_its_lanczos(model, L, chi, monkeypatch):
     """The k range of every y block cut into slots (CT_STAGE3=split) against the tasks: the matvec, and the
-    Lanczos recurrence whose step adds the slots and takes alpha from the tiles' partials."""
+    Lanczos recurrence whose step adds the slots and takes alpha from the tiles' partials (at 1200 states several
+    reduction items per wavefront)."""
     monkeypatch.setenv("CT_STAGE12", "separate")
     p = ct.generate_matvec_problem(model, L, chi, 11)
     got = {}

@@ -3,6 +3,7 @@ lengths and bond dimensions, every operand index of the grouped stages, the colu
 and the fused stages 1 and 2 lies inside its buffer, and every entry of T1, T2 and the result is
 written by exactly one output."""
 
+import numpy as np
 import pytest
 
 import chemtensor_amd as ct
@@ -41,3 +42,17 @@ def test_plan_tables_molecular(n, chi):
     om = orc.MPOView(m.ptr, m.nsites, m.d, m.qsite)
     theta, h2, left, right = orc.matvec_problem_mpo(om, orc.encode_pair(n, 0), chi, 2024)
     assert ct.matvec_plan_check(theta, h2, left, right) == 0
+
+
+def one_sector(da, db, d, D):
+    """theta, h2, left, right with one sector on every axis."""
+    z = lambda n: np.zeros(n, dtype=np.int32)
+    shapes = [(da, d, db), (D, d, d, D), (1, da, D, da), (db, D, db, 1)]
+    dirs = [[1, 1, -1], [1, 1, -1, -1], [1, -1, -1, 1], [1, 1, -1, -1]]
+    return [ct.HostTensor.zeros(s, ad, [z(n) for n in s]) for s, ad in zip(shapes, dirs)]
+
+
+def test_lanczos_step_of_long_vectors():
+    """A vector of four million entries: the workgroups of a Lanczos step on the split stage 3 stay few
+    enough that their reads of the partial sums do not grow with the square of the length."""
+    assert ct.matvec_plan_check(*one_sector(2000, 2000, 1, 1)) == 0
