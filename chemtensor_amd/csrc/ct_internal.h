@@ -263,6 +263,8 @@ struct DevGemm
 	int use_lds = 0;       // one of TileUse
 	// tiles: with the item lists of the LDS-tiled form (plans that time their forms)
 	void upload(const GemmBatch& b, hipStream_t s, bool tiles = false);
+	// only the terms and the tiles of every task (aitems)
+	void upload_tiles(const GemmBatch& b, hipStream_t s);
 	void release();
 };
 constexpr int LDS_TILE = 64;       // output tile edge of the LDS-tiled form
@@ -567,12 +569,24 @@ struct Stage3Split
 {
 	DevGemm g;
 	PairPlan sum;          // partial blocks and reduction items (nunits: tiles)
-	bool ok = false;       // the tables are there
+	GemmBatch batch;       // the host tables from plan to upload
+	std::vector<PrRed> red;
+	bool planned = false;  // the host tables are there
+	bool ok = false;       // the device tables and the partial blocks are there
 	bool use = false;      // the faster of the two ways to run stage 3
 	bool use_lanczos = false;   // the faster one in a Lanczos step, whose update adds the slots itself
-	void build(const GemmBatch& s3, hipStream_t s);
+	void plan(const GemmBatch& s3, int64_t t2_elems);
+	void upload(hipStream_t s);   // not ok when the device memory does not suffice
 	void release();
 };
+// k-panels per slot, 0 where stage 3 is not cut. From S3_TILES tiles per compute unit on the tiles fill the
+// six workgroups that one holds (units and sums against tasks, whole matvec: Hubbard 2000 states, 5.6 tiles
+// per unit, 360 against 352 us; XXZ 2000, 4.1, 850 against 837; XXZ 1000, 1.2, 155 against 159; XXZ 515, 0.4,
+// 50 against 56). The partial blocks, which grow with the height of the blocks (XXZ 4000 states: three
+// times T2), stay within T2 or S3_PART_MIN entries (32 MiB) through longer slots.
+constexpr int S3_TILES = 6;
+constexpr int64_t S3_PART_MIN = (int64_t)1 << 22;
+int stage3_panels(const GemmBatch& s3, int64_t t2_elems, int cus);
 // the slots' tasks (C: element offsets of the partial blocks, pad: the block's first index in y) and the
 // reduction items of a stage-3 batch; false where the tiled form does not apply
 bool split_stage3(const GemmBatch& s3, int panels, GemmBatch& out, std::vector<PrRed>& red, int64_t& part_elems);

@@ -187,8 +187,29 @@ void DevGemm::upload(const GemmBatch& b, hipStream_t s, bool tiles)
 	avg_steps = avg;
 }
 
+void DevGemm::upload_tiles(const GemmBatch& b, hipStream_t s)
+{
+	release();
+	std::vector<WorkItem> ait, none;
+	tile_layout = tile_layout_of(b);
+	split_lds_items(b, {}, 1, ait, none);
+	const size_t n_terms = b.terms.size() * sizeof(GemmTerm), n_ait = ait.size() * sizeof(WorkItem);
+	const size_t o_ait = (std::max<size_t>(n_terms, 1) + 255) / 256 * 256;
+	buf = (char*)dev_alloc(o_ait + std::max<size_t>(n_ait, 1));
+	terms = (GemmTerm*)buf;
+	aitems = (WorkItem*)(buf + o_ait);
+	ntasks = (int)b.tasks.size();
+	nterms = (int)b.terms.size();
+	naitems = (int)ait.size();
+	flops = b.flops;
+	const H2DPart parts[2] = { { b.terms.data(), n_terms, 0 }, { ait.data(), n_ait, o_ait } };
+	copy_h2d_parts(buf, parts, 2, o_ait + n_ait, s);
+}
+
 // k-panels of a term in the LDS-tiled form
 static int64_t term_panels(const GemmTerm& m) { return (m.K + 15) / 16; }
+// slots of a task of 'total' k-panels, about 'panels' each
+static int64_t stage3_slots(int64_t total, int64_t panels) { return std::max<int64_t>(1, (total + panels / 2) / panels); }
 
 bool split_stage3(const GemmBatch& s3, int panels, GemmBatch& out, std::vector<PrRed>& red, int64_t& part_elems)
 {
@@ -199,7 +220,7 @@ bool split_stage3(const GemmBatch& s3, int panels, GemmBatch& out, std::vector<P
 		if (t.sc_i != t.N || y0 + size > INT32_MAX || size > INT32_MAX) return false;
 		int64_t total = 0;
 		for (int q = t.t0; q < t.t1; q++) total += term_panels(s3.terms[(size_t)q]);
-		const int64_t nslots = total > 0 ? std::max<int64_t>(1, (total + panels / 2) / panels) : 0;
+		const int64_t nslots = total > 0 ? stage3_slots(total, panels) : 0;
 		// slot i: panels [total i / nslots, total (i + 1) / nslots) of the task's terms in order
 		int q = t.t0;
 		int64_t q0 = 0;   // panels before term q
@@ -227,38 +248,71 @@ bool split_stage3(const GemmBatch& s3, int panels, GemmBatch& out, std::vector<P
 	return true;
 }
 
-void Stage3Split::build(const GemmBatch& s3, hipStream_t s)
+int stage3_panels(const GemmBatch& s3, int64_t t2_elems, int cus)
 {
-	release();
 	// three tiles per compute unit where the work allows it: slots of at least 6 panels (XXZ bond of 515
 	// states, units and sums: 6 panels 24.6 us, 8 26.8, 16 29.0; 4 panels 26.4) and of at most 24 (molecular
 	// operator, 20 orbitals: 24 panels 205 us, 16 212, 8 240), beyond which only the partial blocks shrink
-	int64_t total = 0;
-	for (const GemmTask& t : s3.tasks) {
-		int64_t tp = 0;
-		for (int q = t.t0; q < t.t1; q++) tp += term_panels(s3.terms[(size_t)q]);
-		total += tp * ((t.M + LDS_TILE - 1) / LDS_TILE) * ((t.N + LDS_TILE - 1) / LDS_TILE);
+	int64_t total = 0, tiles = 0, longest = 0;
+	std::vector<int64_t> task_panels(s3.tasks.size(), 0);
+	for (size_t ti = 0; ti < s3.tasks.size(); ti++) {
+		const GemmTask& t = s3.tasks[ti];
+		for (int q = t.t0; q < t.t1; q++) task_panels[ti] += term_panels(s3.terms[(size_t)q]);
+		const int64_t n = (int64_t)((t.M + LDS_TILE - 1) / LDS_TILE) * ((t.N + LDS_TILE - 1) / LDS_TILE);
+		total += task_panels[ti] * n;
+		tiles += n;
+		longest = std::max(longest, task_panels[ti]);
 	}
-	const int panels = (int)std::min<int64_t>(24, std::max<int64_t>(6, total / (3 * num_compute_units())));
-	GemmBatch b;
-	std::vector<PrRed> red;
-	int64_t elems = 0;
-	if (!split_stage3(s3, panels, b, red, elems)) return;
-	g.upload(b, s, true);
-	sum.red = (PrRed*)dev_alloc(std::max<size_t>(1, red.size()) * sizeof(PrRed));
-	copy_h2d_async(sum.red, red.data(), red.size() * sizeof(PrRed), s);
-	sum.nred = (int)red.size();
-	sum.part = (double*)dev_alloc((size_t)std::max<int64_t>(1, elems) * sizeof(double));
-	sum.part_elems = elems;
-	sum.nunits = g.naitems;
-	ok = true;
+	if (tiles >= S3_TILES * (int64_t)cus) return 0;
+	int64_t panels = std::min<int64_t>(24, std::max<int64_t>(6, total / (3 * cus)));
+	for (;; panels *= 2) {
+		int64_t elems = 0;
+		for (size_t ti = 0; ti < s3.tasks.size(); ti++)
+			elems += (task_panels[ti] > 0 ? stage3_slots(task_panels[ti], panels) : 0) * s3.tasks[ti].M * s3.tasks[ti].N;
+		if (elems <= std::max(S3_PART_MIN, t2_elems)) return (int)panels;
+		if (panels > longest) return 0;
+	}
+}
+
+void Stage3Split::plan(const GemmBatch& s3, int64_t t2_elems)
+{
+	release();
+	const int panels = stage3_panels(s3, t2_elems, num_compute_units());
+	if (panels > 0) planned = split_stage3(s3, panels, batch, red, sum.part_elems);
+	if (!planned) release();
+}
+
+void Stage3Split::upload(hipStream_t s)
+{
+	if (!planned) return;
+	try {
+		g.upload_tiles(batch, s);
+		sum.red = (PrRed*)dev_alloc(std::max<size_t>(1, red.size()) * sizeof(PrRed));
+		copy_h2d_async(sum.red, red.data(), red.size() * sizeof(PrRed), s);
+		sum.nred = (int)red.size();
+		sum.part = (double*)dev_alloc((size_t)std::max<int64_t>(1, sum.part_elems) * sizeof(double));
+		sum.nunits = g.naitems;
+		ok = true;
+	}
+	catch (const HipError& e) {
+		// the plan does without where the device memory is short
+		if (e.code != hipErrorOutOfMemory) throw;
+		(void)hipGetLastError();
+		release();
+	}
+	batch = GemmBatch();
+	red.clear();
+	red.shrink_to_fit();
+	planned = false;
 }
 
 void Stage3Split::release()
 {
 	g.release();
 	sum.release();
-	ok = use = use_lanczos = false;
+	batch = GemmBatch();
+	red.clear();
+	planned = ok = use = use_lanczos = false;
 }
 
 void launch_stage3_units(const Stage3Split& sp, GemmBases b, hipStream_t s, const double* x, double* udot)
@@ -1040,11 +1094,14 @@ int check_grouped_tables(const Meta& th, const Meta& W, const Meta& L, const Met
 	// block's slots, every k of a block in one of them; the workgroups of a Lanczos step on it, each of which
 	// reads the partials of all tiles and workgroups, read them at most four times as often as the vectors and
 	// partial blocks have entries (2^24 reads, about a microsecond, at any size)
-	for (const int panels : { 1, 6, 24 }) {
+	const int chosen = stage3_panels(g.s3, g.t2_elems, 256);
+	for (const int panels : { 1, 6, 24, chosen }) {
+		if (panels == 0) continue;
 		GemmBatch sp;
 		std::vector<PrRed> red;
 		int64_t elems = 0;
 		if (!split_stage3(g.s3, panels, sp, red, elems)) continue;
+		if (panels == chosen && elems > std::max(S3_PART_MIN, g.t2_elems)) return 12;
 		std::vector<int> wp((size_t)elems, 0), wr((size_t)th.nelem, 0);
 		if (!check_batch(sp, L.nelem, g.t2_elems, elems, &wp) || !once(wp)) return 9;
 		int64_t k0 = 0, k1 = 0;
@@ -1168,7 +1225,7 @@ static void build_grouped(MatvecPlan& p, bool lean)
 	p.stage[1].upload(g.s2, p.stream, tiles);
 	p.stage[2].upload(g.s3, p.stream, tiles);
 	for (int i = 0; i < 3; i++) p.stage_bytes[i] = g.stage_bytes[i];
-	if (tiles) p.split3.build(g.s3, p.stream);
+	if (tiles) p.split3.plan(g.s3, g.t2_elems);
 	p.stage_flops[0] = g.s1.flops;
 	p.stage_flops[1] = g.s2.flops;
 	p.stage_flops[2] = g.s3.flops;
@@ -1338,6 +1395,8 @@ void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, 
 		}
 		if (st == 0) best1 = best;
 		if (st == 1) best2 = best;
+		// after every other allocation of the plan, whose memory it must not take
+		if (st == 2 && split3) split3->upload(s);
 		if (st == 2 && split3 && split3->ok) {
 			const float ms = time3([&] { launch_stage3_units(*split3, b, s); launch_pair_reduce(split3->sum, y, s); });
 			split3->use = ms < best;
@@ -1346,6 +1405,7 @@ void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, 
 			const char* force = getenv("CT_STAGE3");
 			if (force && strcmp(force, "tasks") == 0) split3->use = split3->use_lanczos = false;
 			if (force && strcmp(force, "split") == 0) split3->use = split3->use_lanczos = true;
+			if (!split3->use && !split3->use_lanczos) split3->release();
 		}
 	}
 	if (use_wapply) {
@@ -1427,6 +1487,7 @@ void launch_grouped_stages(const DevGemm* stage, const GemmBases* bases, const W
 static void autotune_stages(MatvecPlan& p)
 {
 	autotune_grouped(p.stage, p.stage_bases, &p.wapply, &p.use_wapply, &p.use_f12, &p.wtiles, &p.split3, p.theta_meta.nelem, p.stream, p.tuned_ms);
+	if (p.split3.ok) p.interm_elems += (double)p.split3.sum.part_elems;
 	if (p.use_f12 && p.wapply.f12_ok) {
 		// one launch for stages 1 and 2: theta, R and W in, T2 out (T1 never written)
 		const double t1 = (double)p.interm[0].meta.nelem;

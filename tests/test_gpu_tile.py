@@ -86,6 +86,23 @@ def test_split_stage3_and_its_lanczos(model, L, chi, monkeypatch):
     assert np.linalg.norm(a[2] - b[2]) <= 1e-10
 
 
+@pytest.mark.parametrize("model,L,chi", [("hubbard", 8, 24), ("xxz", 20, 64)])
+def test_partial_blocks_only_where_used(model, L, chi, monkeypatch):
+    """A plan keeps the split's partial blocks (in its intermediate doubles) only where stage 3 runs on them:
+    vectors this short do not take them into the Lanczos step."""
+    p = ct.generate_matvec_problem(model, L, chi, 11)
+    held = {}
+    for stage3 in ("tasks", "split", None):
+        if stage3:
+            monkeypatch.setenv("CT_STAGE3", stage3)
+        else:
+            monkeypatch.delenv("CT_STAGE3")
+        plan = ct.MatvecPlan(*p, ct.GROUPED_FP64)
+        held[stage3] = (plan.forms()[0][2], plan.stats()["intermediate_doubles"])
+    assert held["split"][0] == 7 and held["split"][1] > held["tasks"][1]
+    assert held[None][1] == held["split" if held[None][0] == 7 else "tasks"][1]
+
+
 @pytest.mark.parametrize("density", [0.0, 0.02, 0.3, 1.0])
 @pytest.mark.parametrize("da,db,d,D", [(1, 1, 2, 20), (3, 5, 4, 17), (17, 9, 2, 33), (5, 64, 3, 48), (33, 2, 2, 65), (1, 129, 1, 40)])
 def test_row_tiles_of_wide_classes(da, db, d, D, density, monkeypatch):

@@ -56,3 +56,9 @@ def test_lanczos_step_of_long_vectors():
     """A vector of four million entries: the workgroups of a Lanczos step on the split stage 3 stay few
     enough that their reads of the partial sums do not grow with the square of the length."""
     assert ct.matvec_plan_check(*one_sector(2000, 2000, 1, 1)) == 0
+
+
+@pytest.mark.parametrize("da,db", [(6000, 60), (5000, 90)])
+def test_partial_blocks_of_high_blocks(da, db):
+    """Few high blocks: the partial blocks of the split stage 3 stay within T2 or 32 MiB (code 12)."""
+    assert ct.matvec_plan_check(*one_sector(da, db, 1, 1)) == 0
