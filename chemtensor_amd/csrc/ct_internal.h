@@ -594,17 +594,21 @@ bool split_stage3(const GemmBatch& s3, int panels, GemmBatch& out, std::vector<P
 void launch_stage3_units(const Stage3Split& sp, GemmBases b, hipStream_t s, const double* x = nullptr, double* udot = nullptr);
 
 // A Lanczos step on the split stage 3 has one launch less than on the tasks (the step adds the slots, the
-// tiles write the alpha partials): worth LZ_SAVED_MS (ms) between vectors of LZ_SPLIT_MIN and of LZ_SPLIT_MAX
-// entries. 20 steps on sweep-like bonds, tasks against split, beside the time that the split takes more or
-// less for one matvec: XXZ 250 states (59000 entries) 716 against 631 us, -1 us; 515 states (272000) 1403
-// against 1219, -6; 1000 states (983000) 3505 against 3414, -4; Hubbard 512 states (245000) 963 against 948,
-// +2; 1000 states (952000) 2128 against 2223, +8. Beyond, a wavefront adds the slots of several items one
-// after another: XXZ 2000 states (3974000) 17800 against 18400, Hubbard 2000 states (3606000) 8020 against
-// 8400. Below, at 2000 to 15000 entries, 427 against 418 and 478 against 472, hardly more than two runs
-// differ by. The two ways round differently at every size: Ritz vectors by 1e-15 on random environments, by
-// 1e-14 on sweep-like ones, with the same sign in 48 pairs of solves of 1 to 20 steps, 240 to 116000 entries.
-constexpr float LZ_SAVED_MS = 0.003f;
-constexpr int64_t LZ_SPLIT_MIN = (int64_t)1 << 15, LZ_SPLIT_MAX = (int64_t)1 << 20;
+// tiles write the alpha partials): the time (ms) by which stage 3 may be slower on the split for vectors of n
+// entries. Measured on 16 bonds, stage 3 on tasks and split, then 20 steps on tasks and split (us): up to
+// 2^18 entries the step saves 4 to 5.6 (Hubbard 300 states, 86000 entries, 7.7 and 11.9, 738 and 714; 512
+// states, 245000, 11.5 and 15.5, 977 and 944; XXZ 300, 93000, 11.4 and 12.1, 828 and 730), above 1 to 4
+// (Hubbard 700, 460000, 19.2 and 24.4, 1327 and 1409; XXZ 515, 272000, 27.5 and 24.0, 1438 and 1257; XXZ 1000,
+// 983000, 71.6 and 69.8, 3542 and 3442). Beyond 2^20 a wavefront of the step adds the slots of several items
+// one after another (XXZ 2000, 3974000, 17800 and 18400; Hubbard 2000, 3606000, 8020 and 8400), and at 2000
+// to 15000 entries 427 against 418 and 478 against 472 are hardly more than two runs differ by. The two ways
+// round differently at every size: Ritz vectors by 1e-15 on random environments, by 1e-14 on sweep-like ones,
+// with the same sign in 48 pairs of solves of 1 to 20 steps, 240 to 116000 entries.
+inline float lz_split_saved_ms(int64_t n)
+{
+	if (n < (int64_t)1 << 15 || n > (int64_t)1 << 20) return -1e30f;
+	return n <= (int64_t)1 << 18 ? 0.0045f : 0.0025f;
+}
 
 struct MatvecPlan
 {

@@ -1400,7 +1400,7 @@ void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, 
 		if (st == 2 && split3 && split3->ok) {
 			const float ms = time3([&] { launch_stage3_units(*split3, b, s); launch_pair_reduce(split3->sum, y, s); });
 			split3->use = ms < best;
-			split3->use_lanczos = nx >= LZ_SPLIT_MIN && nx <= LZ_SPLIT_MAX && ms - best < LZ_SAVED_MS;
+			split3->use_lanczos = ms - best < lz_split_saved_ms(nx);
 			// CT_STAGE3=split|tasks overrides the timing-based choice
 			const char* force = getenv("CT_STAGE3");
 			if (force && strcmp(force, "tasks") == 0) split3->use = split3->use_lanczos = false;
