@@ -360,8 +360,9 @@ __global__ __launch_bounds__(256) void k_pair_reduce_dot(const PrRed* __restrict
 // Every workgroup reads all the partials, so at one item per wavefront their traffic would grow with the
 // square of the vector length (Hubbard bond of 2000 states, 3.6e6 entries: 14133 workgroups reading 17352
 // partials each, 2 GB; 20 steps 9870 us, 8400 us with the limit): beyond PR_STEP_GRID workgroups a wavefront
-// takes several items in turn, the first one's loads ahead of the partials.
+// takes several items in turn, the first one's loads ahead of the partials (MANY).
 constexpr int PR_STEP_GRID = 2048;
+template <bool MANY>
 __global__ __launch_bounds__(256) void k_pair_lz_step(const PrRed* __restrict__ items, const int nitems, const double* __restrict__ part,
 	const double* __restrict__ uj, double* __restrict__ unext, double* __restrict__ vj_out, const double* __restrict__ vjm1, int j, int maxiter,
 	const double* __restrict__ dpart, int Gd, const double* __restrict__ npart, int Gn, double thresh, double* __restrict__ npart_out,
@@ -446,6 +447,7 @@ __global__ __launch_bounds__(256) void k_pair_lz_step(const PrRed* __restrict__ 
 				acc += wi * wi;
 			}
 		}
+		if constexpr (!MANY) break;
 		w += 4 * (int)gridDim.x;
 		if (w >= nitems) break;
 		load();
@@ -1357,7 +1359,8 @@ void launch_pair_lz_step(const PairPlan& pp, const double* uj, double* unext, do
 	const double* dpart, const double* npart, double thresh, double* npart_out, double* scal, hipStream_t s)
 {
 	const int G = pair_step_grid(pp.nred);
-	hipLaunchKernelGGL(k_pair_lz_step, dim3((unsigned)G), dim3(256), 0, s, (const PrRed*)pp.red, pp.nred, (const double*)pp.part, uj, unext, vj_out, vjm1,
+	const auto kernel = pp.nred > 4 * G ? k_pair_lz_step<true> : k_pair_lz_step<false>;
+	hipLaunchKernelGGL(kernel, dim3((unsigned)G), dim3(256), 0, s, (const PrRed*)pp.red, pp.nred, (const double*)pp.part, uj, unext, vj_out, vjm1,
 		j, maxiter, dpart, std::max(0, pp.nunits), npart, G, thresh, npart_out, scal);
 	CTG_HIP(hipGetLastError());
 }
