@@ -1362,6 +1362,10 @@ void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, 
 		CTG_HIP(hipEventElapsedTime(&ms, e0, e1));
 		return ms / 3;
 	};
+	// CT_GEMM_LDS overrides the timing-based choice of the LDS-tiled form: 0 never (nor the split stage 3, which
+	// runs on its tiles), 1 the faster of the large tasks and every task, large | all that one where a stage has it
+	const char* lds = getenv("CT_GEMM_LDS");
+	const bool lds_off = lds && lds[0] == '0';
 	float best1 = 1e30f, best2 = 1e30f;
 	for (int st = 0; st < 3; st++) {
 		DevGemm& g = stage[st];
@@ -1377,19 +1381,18 @@ void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, 
 			if (ms < best) { best = ms; best_form = f; }
 		}
 		g.form = best_form;
-		// the large tasks on the LDS-tiled form and the rest on the best form, or every task on the LDS-tiled
-		// form (CT_GEMM_LDS=0|1: never / the faster of the two, whatever the others take)
+		// the large tasks on the LDS-tiled form and the rest on the best form, or every task on the LDS-tiled form
 		if (g.nlitems > 0 || g.naitems > 0) {
 			float tile_best = 1e30f;
 			int tile_use = TILE_NONE;
 			for (const int use : { TILE_LARGE, TILE_ALL }) {
 				if (use == TILE_LARGE ? g.nlitems == 0 : g.naitems == 0) continue;
+				if (lds && strcmp(lds, use == TILE_LARGE ? "all" : "large") == 0) continue;
 				g.use_lds = use;
 				const float ms = time3([&] { launch_grouped_gemm_f64(g, b, s); });
 				if (ms < tile_best) { tile_best = ms; tile_use = use; }
 			}
-			const char* force = getenv("CT_GEMM_LDS");
-			const bool use = force && force[0] == '0' ? false : force && force[0] == '1' ? true : tile_best < best;
+			const bool use = tile_use != TILE_NONE && (lds ? !lds_off : tile_best < best);
 			g.use_lds = use ? tile_use : TILE_NONE;
 			if (use && tile_best < best) best = tile_best;
 		}
@@ -1401,6 +1404,7 @@ void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, 
 			const float ms = time3([&] { launch_stage3_units(*split3, b, s); launch_pair_reduce(split3->sum, y, s); });
 			split3->use = ms < best;
 			split3->use_lanczos = ms - best < lz_split_saved_ms(nx);
+			if (lds_off) split3->use = split3->use_lanczos = false;
 			// CT_STAGE3=split|tasks overrides the timing-based choice
 			const char* force = getenv("CT_STAGE3");
 			if (force && strcmp(force, "tasks") == 0) split3->use = split3->use_lanczos = false;

@@ -124,8 +124,9 @@ def test_molecular_matvec_forms_match_oracle(n, chi):
 @pytest.mark.parametrize("n,chi", [(12, 128), (20, 512)])
 def test_molecular_matvec_lds_form(n, chi, monkeypatch):
     """The LDS-tiled GEMM form (64 x 64 workgroup tiles for the large tasks of the molecular
-    operator) forced on and off, against the oracle at 1e-12 and against each other (the forms
-    chosen without it split the k-steps of a tile differently, so the sums agree to rounding)."""
+    operator) forced on and off in every stage (stage 2 as MFMA products), against the oracle at
+    1e-12 and against each other (the forms chosen without it split the k-steps of a tile
+    differently, so the sums agree to rounding)."""
     from oracle import oracle as orc
     t, v = ct.molecular_coefficients(n, 5)
     pm = ct.MPO.spin_molecular(t, v)
@@ -134,6 +135,7 @@ def test_molecular_matvec_lds_form(n, chi, monkeypatch):
     want = orc.apply_local_hamiltonian(theta, h2, left, right).serialize()
     x = ct.DeviceArray.from_numpy(theta.serialize())
     ys = {}
+    monkeypatch.setenv("CT_STAGE2", "mfma")
     for lds in ("1", "0"):
         monkeypatch.setenv("CT_GEMM_LDS", lds)
         plan = ct.MatvecPlan(theta, h2, left, right, ct.GROUPED_FP64)
@@ -146,5 +148,7 @@ def test_molecular_matvec_lds_form(n, chi, monkeypatch):
         say("molecular n", n, "CT_GEMM_LDS", lds, "forms", list(forms), "rel err", err)
         assert err < 1e-12
         if lds == "1":
-            assert 6 in list(forms)
+            assert forms[1] == 6
+        else:
+            assert not {6, 7, 8} & set(forms)
     assert np.max(np.abs(ys["1"] - ys["0"])) < 1e-13 * np.max(np.abs(ys["0"]))

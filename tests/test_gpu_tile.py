@@ -103,6 +103,42 @@ def test_partial_blocks_only_where_used(model, L, chi, monkeypatch):
     assert held[None][1] == held["split" if held[None][0] == 7 else "tasks"][1]
 
 
+def test_tiles_off(monkeypatch):
+    """CT_GEMM_LDS=0: no stage on the LDS tiles, neither as tasks nor as slots of a cut k range (a bond that
+    takes both without the switch)."""
+    p = ct.generate_matvec_problem("xxz", 32, 256, 11)
+    monkeypatch.setenv("CT_STAGE12", "separate")
+    monkeypatch.setenv("CT_STAGE3", "tasks")
+    tasks = ct.MatvecPlan(*p, ct.GROUPED_FP64).stats()["intermediate_doubles"]
+    monkeypatch.delenv("CT_STAGE3")
+    monkeypatch.setenv("CT_GEMM_LDS", "0")
+    plan = ct.MatvecPlan(*p, ct.GROUPED_FP64)
+    assert not {6, 7} & set(plan.forms()[0]) and plan.stats()["intermediate_doubles"] == tasks
+
+
+@pytest.mark.parametrize("which", ["large", "all"])
+@pytest.mark.parametrize("model,chi", [("hubbard", 1600), ("xxz", 515)])
+def test_tiles_of_large_and_of_all_tasks(model, chi, which, monkeypatch):
+    """Bonds with tasks on both sides of the limit: the large ones on the tiles and the others on the wavefront
+    forms in a second launch, or all on the tiles, against the wavefront forms alone."""
+    p = ct.generate_matvec_problem(model, 32, chi, 11)
+    monkeypatch.setenv("CT_STAGE12", "separate")
+    monkeypatch.setenv("CT_STAGE3", "tasks")
+    x, got = ct.DeviceArray.from_numpy(p[0].serialize()), {}
+    for lds in ("0", which):
+        monkeypatch.setenv("CT_GEMM_LDS", lds)
+        plan = ct.MatvecPlan(*p, ct.GROUPED_FP64)
+        forms = plan.forms()[0]
+        print("case", model, chi, lds, "forms", forms, flush=True)
+        assert (forms[0] == 6 and forms[2] == 6) == (lds != "0")
+        y = ct.DeviceArray(plan.dim)
+        plan.apply(x, y)
+        plan.synchronize()
+        got[lds] = y.numpy()
+    # the same products, added in an order of their own in some of the wavefront forms
+    assert np.linalg.norm(got["0"] - got[which]) <= 1e-14 * np.linalg.norm(got["0"])
+
+
 @pytest.mark.parametrize("density", [0.0, 0.02, 0.3, 1.0])
 @pytest.mark.parametrize("da,db,d,D", [(1, 1, 2, 20), (3, 5, 4, 17), (17, 9, 2, 33), (5, 64, 3, 48), (33, 2, 2, 65), (1, 129, 1, 40)])
 def test_row_tiles_of_wide_classes(da, db, d, D, density, monkeypatch):
