@@ -153,3 +153,39 @@ def test_row_tiles_of_wide_classes(da, db, d, D, density, monkeypatch):
     plan.apply(x, y)
     plan.synchronize()
     assert np.linalg.norm(y.numpy() - want) <= 2e-14 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("da,db,d,D", [(2, 50, 2, 33), (3, 49, 2, 24), (17, 9, 2, 33), (5, 64, 3, 48), (33, 2, 2, 65), (7, 31, 1, 129)])
+def test_tiles_of_several_column_runs(da, db, d, D, monkeypatch):
+    """Stage 2 of a wide operator as products whose columns lie in several runs, one per row of the block pair:
+    the 64 x 64 tiles that read any layout."""
+    monkeypatch.setenv("CT_STAGE2", "mfma")
+    monkeypatch.setenv("CT_GEMM_LDS", "large")
+    ts, want = dense_problem(da, db, d, D, 5 * da + db)
+    plan = ct.MatvecPlan(*ts, ct.GROUPED_FP64)
+    print("case", da, db, d, D, "forms", plan.forms()[0], flush=True)
+    assert plan.forms()[0][1] == 6
+    x, y = ct.DeviceArray.from_numpy(ts[0].serialize()), ct.DeviceArray(plan.dim)
+    plan.apply(x, y)
+    plan.synchronize()
+    assert np.linalg.norm(y.numpy() - want) <= 2e-14 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("stage2", ["rowtiles", "mfma"])
+@pytest.mark.parametrize("n,chi", [(8, 96), (8, 150), (10, 160)])
+def test_wide_classes_of_several_sectors(n, chi, stage2, monkeypatch):
+    """Stage 2 of a molecular operator, with classes of many sectors and blocks that are absent, as row tiles and
+    as tiles that read any layout, against the oracle."""
+    from oracle import oracle as orc
+    monkeypatch.setenv("CT_STAGE2", stage2)
+    monkeypatch.setenv("CT_GEMM_LDS", "large")
+    pm = ct.MPO.spin_molecular(*ct.molecular_coefficients(n, 5))
+    p = orc.matvec_problem_mpo(orc.MPOView(pm.ptr, pm.nsites, pm.d, pm.qsite), orc.encode_pair(n, 0), chi, 2024)
+    want = orc.apply_local_hamiltonian(*p).serialize()
+    plan = ct.MatvecPlan(*p, ct.GROUPED_FP64)
+    print("case", n, chi, stage2, "forms", plan.forms()[0], flush=True)
+    assert plan.forms()[0][1] == (8 if stage2 == "rowtiles" else 6)
+    x, y = ct.DeviceArray.from_numpy(p[0].serialize()), ct.DeviceArray(plan.dim)
+    plan.apply(x, y)
+    plan.synchronize()
+    assert np.linalg.norm(y.numpy() - want) <= 2e-14 * np.linalg.norm(want)
