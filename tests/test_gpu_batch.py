@@ -63,12 +63,20 @@ def test_batched_lanczos_matches_single_plans(problems, form, monkeypatch):
     rng = np.random.default_rng(11)
     v0 = rng.standard_normal(batch.dim)
     maxiter = 15
-    lam_g, st_g, u_g = batch.lanczos(ct.DeviceArray.from_numpy(v0), maxiter)
+    starts = [v0, rng.standard_normal(batch.dim)]
     monkeypatch.setenv("CT_LANCZOS_GRAPH", "0")
-    lam_e, st_e, u_e = batch.lanczos(ct.DeviceArray.from_numpy(v0), maxiter)
-    assert np.array_equal(st_g, np.zeros(len(problems))) and np.array_equal(st_e, st_g)
-    assert np.array_equal(lam_g, lam_e)                      # graph replay == eager launches
-    assert np.array_equal(u_g.numpy(), u_e.numpy())
+    eager = [batch.lanczos(ct.DeviceArray.from_numpy(v), maxiter) for v in starts]
+    monkeypatch.delenv("CT_LANCZOS_GRAPH")
+    x, y = ct.DeviceArray.from_numpy(v0), ct.DeviceArray(batch.dim)
+    # an eager solve, the captured one, replays; eager work and a synchronisation between them
+    for which in (0, 0, 1, 0, 1, 0):
+        lam_g, st_g, u_g = batch.lanczos(ct.DeviceArray.from_numpy(starts[which]), maxiter)
+        lam_e, st_e, u_e = eager[which]
+        assert np.array_equal(st_g, np.zeros(len(problems))) and np.array_equal(st_e, st_g)
+        assert np.array_equal(lam_g, lam_e)                  # graph replay == eager launches
+        assert np.array_equal(u_g.numpy(), u_e.numpy())
+        batch.apply(x, y)
+        batch.synchronize()
     ug = u_g.numpy()
     for i, p in enumerate(problems):
         plan = ct.MatvecPlan(*p[:4], ct.FUSED_FP64)

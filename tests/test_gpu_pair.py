@@ -85,7 +85,7 @@ def test_pair_lanczos_matches_grouped():
     plan = ct.MatvecPlan(theta, h2, left, right, ct.PAIR_FP64)
     import os
     vals = []
-    for flag in ("1", "1", "0"):
+    for flag in ("1", "1", "1", "0"):      # eager, captured, replayed, eager
         os.environ["CT_LANCZOS_GRAPH"] = flag
         lam, u = plan.lanczos(v0, 20)
         vals.append((lam, u.numpy()))
@@ -117,7 +117,7 @@ def test_pair_lanczos_step_from_partials(model, L, chi, monkeypatch):
     monkeypatch.setenv("CT_PAIR_LZ_FUSED", "1")
     plan = ct.MatvecPlan(theta, h2, left, right, ct.PAIR_FP64)
     vals = []
-    for flag in ("1", "1", "0"):
+    for flag in ("1", "1", "1", "0"):      # eager, captured, replayed, eager
         monkeypatch.setenv("CT_LANCZOS_GRAPH", flag)
         lam, u = plan.lanczos(v0, 16)
         vals.append((lam, u.numpy()))
