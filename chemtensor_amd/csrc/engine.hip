@@ -8,6 +8,7 @@
 #include <map>
 #include <cstring>
 #include <numeric>
+#include <set>
 #include <unordered_map>
 
 #include "ct_internal.h"
@@ -1119,27 +1120,61 @@ int check_grouped_tables(const Meta& th, const Meta& W, const Meta& L, const Met
 	}
 	const WApplyHost& wa = g.wa;
 	if (wa.kmax > WA_KMAX) {
-		// the row tiles of an operator with one entry in five: every T2 entry written once, every non-zero
-		// entry of W in one pack, and in a sub-tile that its panel's mask runs
+		// the row tiles of an operator with one entry in five: every entry of a class of W_D that is not zero at
+		// its place in one pack, in a sub-tile that its panel's mask runs, and zeros elsewhere; the T1 entries of
+		// every kept column inside the item's range of T1; every T2 entry written once
 		std::vector<double> wv((size_t)W.nelem, 0.0);
-		size_t nnz = 0, packed = 0;
 		for (size_t i = 0; i < wv.size(); i++) if (i * 2654435761u % 5 == 0) wv[i] = 1.0 + (double)i;
 		WtHost h;
 		if (plan_wtiles(h, wa, W, wv.data())) {
-			for (double v : wv) nnz += v != 0.0;
-			for (size_t i = 0; i < h.pack.size(); i++) {
-				if (h.pack[i] == 0.0) continue;
-				packed++;
-				const size_t p = i / 1024, o = i % 1024, st = o / 256, sub = o / 128 % 2 * 2 + o % 2;
-				if (!(h.masks[p] >> (4 * st + sub) & 1)) return 10;
-			}
-			// entries of W outside every class act on no block
-			if (packed > nnz) return 10;
+			// W_D of a class, entry by entry from the blocks of W
+			auto dense = [&](const WaClass& c) {
+				std::vector<double> m((size_t)c.R * c.K, 0.0);
+				int r = 0;
+				for (const auto& mq : c.rows)
+					for (ct_long i = 0; i < W.block_count[0][mq.first] * W.block_count[1][mq.second]; i++, r++) {
+						int k = 0;
+						for (const auto& pn : c.cols) {
+							const ct_long n = W.block_count[2][pn.first] * W.block_count[3][pn.second];
+							const ct_long iw[4] = { mq.first, mq.second, pn.first, pn.second };
+							const ct_long kw = W.flat_index(iw);
+							for (ct_long j = 0; j < n; j++, k++)
+								if (W.present(kw)) m[(size_t)r * c.K + k] = wv[(size_t)(W.offset[kw] + i * n + j)];
+						}
+					}
+				return m;
+			};
+			std::map<int64_t, int> class_of;                 // by a unit's first column
+			for (size_t ui = 0; ui < wa.units.size(); ui++) class_of[wa.units[ui].kb] = wa.unit_class[ui];
+			std::map<int, std::pair<std::vector<double>, std::vector<uint8_t>>> found;   // of the classes with units: W_D, entries found
+			std::set<int64_t> packs;
 			std::vector<int> ws((size_t)g.t2_elems, 0);
 			for (const WtItem& it : h.items) {
 				const int dCp = (it.dC + 1) & ~1;
-				if (it.np < 1 || it.np * 16 > 2048 || (size_t)(it.klist + 16 * it.np) > h.lists.size() || (size_t)(it.mask + it.np) > h.masks.size() ||
-					(size_t)it.pack + (size_t)it.np * 1024 > h.pack.size() || it.t1_off + it.t1_bytes / 8 > g.t1_elems || it.t2_off + it.t2_bytes / 8 > g.t2_elems) return 10;
+				if (it.np < 1 || it.np * 16 > 2048 || (size_t)(it.klist + 16 * it.np) > h.lists.size() || (size_t)(it.rlist + 64) > h.lists.size() ||
+					(size_t)(it.mask + it.np) > h.masks.size() || (size_t)it.pack + (size_t)it.np * 1024 > h.pack.size() ||
+					it.t1_off + it.t1_bytes / 8 > g.t1_elems || it.t2_off + it.t2_bytes / 8 > g.t2_elems || !class_of.count(it.kb)) return 10;
+				const int ci = class_of[it.kb];
+				const WaClass& c = wa.classes[(size_t)ci];
+				if (!found.count(ci)) found[ci] = { dense(c), std::vector<uint8_t>((size_t)c.R * c.K, 0) };
+				const std::vector<double>& m = found[ci].first;
+				std::vector<uint8_t>& f = found[ci].second;
+				for (int q = 0; q < 16 * it.np; q++) {
+					const int k = h.lists[(size_t)(it.klist + q)];
+					const int64_t b = k >= 0 ? wa.kbase[(size_t)(it.kb + k)] : -1;
+					if (k >= c.K) return 10;
+					if (b >= 0 && (b < it.t1_off || b + (int64_t)(it.dA - 1) * wa.kstride[(size_t)(it.kb + k)] + it.dC > it.t1_off + it.t1_bytes / 8)) return 10;
+				}
+				const bool first = packs.insert(it.pack).second;   // the tile's column tiles share its pack
+				for (int x = 0; first && x < 64; x++)
+					for (int q = 0; q < 16 * it.np; q++) {
+						const int r = h.lists[(size_t)(it.rlist + x)], k = h.lists[(size_t)(it.klist + q)];
+						const double v = h.pack[(size_t)it.pack + (size_t)(q / 16) * 1024 + (size_t)(q % 16 / 4) * 256 + (size_t)(x / 32) * 128 +
+							(size_t)(16 * (q % 4) + x % 16) * 2 + (size_t)(x / 16 % 2)];
+						if (r >= c.R || v != (r >= 0 && k >= 0 ? m[(size_t)r * c.K + k] : 0.0)) return 10;
+						if (v == 0.0) continue;
+						if (!(h.masks[(size_t)(it.mask + q / 16)] >> (4 * (q % 16 / 4) + x / 16) & 1) || f[(size_t)r * c.K + k]++) return 10;
+					}
 				for (int i = 0; i < 64; i++) {
 					const int r = h.lists[(size_t)(it.rlist + i)];
 					const int64_t b = r >= 0 ? wa.rbase[(size_t)(it.rb + r)] : -1;
@@ -1153,6 +1188,9 @@ int check_grouped_tables(const Meta& th, const Meta& W, const Meta& L, const Met
 					}
 				}
 			}
+			for (const auto& fc : found)
+				for (size_t i = 0; i < fc.second.first.size(); i++)
+					if ((fc.second.first[i] != 0.0) != (fc.second.second[i] != 0)) return 10;
 			if (!once(ws)) return 10;
 		}
 	}
