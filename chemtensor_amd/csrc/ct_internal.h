@@ -382,6 +382,7 @@ struct WtHost
 	std::vector<int> lists;        // per tile: 64 rows of the class, then its columns (-1: none)
 	std::vector<uint32_t> masks;   // per panel: bit 4 step + sub-tile
 	std::vector<double> pack;      // per panel: 16 columns x 64 rows in fragment order
+	double flops = 0;              // of the products with entries of W that are not zero
 };
 struct WTiles
 {
@@ -390,6 +391,7 @@ struct WTiles
 	uint32_t* masks = nullptr;
 	double* pack = nullptr;
 	int nitems = 0;
+	double flops = 0;
 	bool ok = false, use = false;
 	void upload(const WtHost& h, hipStream_t s);
 	void release();
@@ -635,7 +637,7 @@ struct MatvecPlan
 	std::vector<void*> owned;                   // device descriptor buffers of the plain form
 	// bookkeeping
 	double flops = 0, bytes = 0;
-	double stage_flops[3] = { 0, 0, 0 };        // executed FP64 flops of each stage
+	double stage_flops[3] = { 0, 0, 0 };        // FP64 flops of each stage, as formed (no tile padding)
 	double stage_bytes[3] = { 0, 0, 0 };        // algorithmic bytes of each stage (operands read once, result written once)
 	float tuned_ms[3][GEMM_NUM_FORMS] = {};     // autotuner timings (ms per launch) of each stage and form
 	double nterms = 0, ntasks = 0, nitems = 0, interm_elems = 0;

@@ -1529,6 +1529,7 @@ void launch_grouped_stages(const DevGemm* stage, const GemmBases* bases, const W
 static void autotune_stages(MatvecPlan& p)
 {
 	autotune_grouped(p.stage, p.stage_bases, &p.wapply, &p.use_wapply, &p.use_f12, &p.wtiles, &p.split3, p.theta_meta.nelem, p.stream, p.tuned_ms);
+	if (p.wtiles.use) p.stage_flops[1] = p.wtiles.flops;   // the products with zeros of W are left out
 	if (p.split3.ok) p.interm_elems += (double)p.split3.sum.part_elems;
 	if (p.use_f12 && p.wapply.f12_ok) {
 		// one launch for stages 1 and 2: theta, R and W in, T2 out (T1 never written)

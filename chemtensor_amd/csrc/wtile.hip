@@ -223,6 +223,7 @@ static void plan_row_tiles(WtHost& h, const std::vector<double>& w, int R, int K
 bool plan_wtiles(WtHost& h, const WApplyHost& wa, const Meta& W, const double* w)
 {
 	std::vector<std::vector<WtTile>> tiles(wa.classes.size());
+	std::vector<int64_t> nonzero(wa.classes.size(), 0);
 	for (size_t ci = 0; ci < wa.classes.size(); ci++) {
 		const WaClass& c = wa.classes[ci];
 		if (c.K > WT_KMAX) return false;
@@ -243,6 +244,7 @@ bool plan_wtiles(WtHost& h, const WApplyHost& wa, const Meta& W, const double* w
 			}
 			r0 += (int)(dM * dQ);
 		}
+		for (const double v : m) nonzero[ci] += v != 0.0;
 		plan_row_tiles(h, m, c.R, c.K, tiles[ci]);
 	}
 	// the tiles of one column tile share its T1 panel: they go to one XCD, the column tiles dealt to the
@@ -278,6 +280,7 @@ bool plan_wtiles(WtHost& h, const WApplyHost& wa, const Meta& W, const double* w
 		q.t2_bytes = (int)b2;
 		int64_t cost = 0;
 		for (const WtTile& t : ts) cost += t.cost;
+		h.flops += 2.0 * (double)nonzero[(size_t)wa.unit_class[ui]] * u.dA * u.dC;
 		const int cols = u.dA * ((u.dC + 1) & ~1);
 		for (int j0 = 0; j0 < cols; j0 += 64) groups.push_back(Group{ cost, ui, j0 });
 	}
@@ -322,6 +325,7 @@ void WTiles::upload(const WtHost& h, hipStream_t s)
 	masks = upload_new(h.masks, s);
 	pack = upload_new(h.pack, s);
 	nitems = (int)h.items.size();
+	flops = h.flops;
 	ok = true;
 }
 

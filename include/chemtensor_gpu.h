@@ -221,7 +221,8 @@ double ct_matvec_plan_flops(const ct_matvec_plan* plan);
 double ct_matvec_plan_bytes(const ct_matvec_plan* plan);
 /// plan statistics: [0] GEMM terms (stage 1,2,3 summed), [1] output tasks, [2] work items, [3] intermediate doubles
 int ct_matvec_plan_stats(const ct_matvec_plan* plan, double* stats4);
-/// per-stage algorithmic flops (stage 1: theta.R, 2: W.T1, 3: L^T.T2) of the grouped forms
+/// per-stage flops (stage 1: theta.R, 2: W.T1, 3: L^T.T2) of the products that the grouped forms form: of whole
+/// blocks, and of the non-zero entries of W where stage 2 runs as row tiles
 int ct_matvec_plan_stage_flops(const ct_matvec_plan* plan, double* flops3);
 /// per-stage algorithmic bytes: 8 (|inputs| + |output|) of each stage's launch
 int ct_matvec_plan_stage_bytes(const ct_matvec_plan* plan, double* bytes3);

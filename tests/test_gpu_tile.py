@@ -150,6 +150,7 @@ def test_row_tiles_of_wide_classes(da, db, d, D, density, monkeypatch):
     plan = ct.MatvecPlan(*ts, ct.GROUPED_FP64)
     print("case", da, db, d, D, density, "forms", plan.forms()[0], flush=True)
     assert plan.forms()[0][1] == 8
+    assert plan.stage_flops()[1] == 2 * np.count_nonzero(ts[1].serialize()) * da * db
     x, y = ct.DeviceArray.from_numpy(ts[0].serialize()), ct.DeviceArray(plan.dim)
     plan.apply(x, y)
     plan.synchronize()
