@@ -26,14 +26,15 @@ struct TilePanel { double2_t a[2], b[2]; };
 
 // One 64 x 64 tile per workgroup of four wavefronts, terms in order and k ascending in steps of four (the
 // order of the wavefront forms). What bounds it: the FP64 matrix rate. A 16x16x4 MFMA holds its SIMD for
-// 64 cycles; vector instructions do not run beside it and a vector memory instruction costs it about 25
+// 64 cycles; vector instructions do not run beside it and a vector memory instruction costs it 25 to 28
 // cycles whatever its width (measured with four wavefronts per SIMD), so the panel loop has as few of both
 // as possible: loads are 16 bytes wide at 8-byte alignment, their per-thread offsets stay the same over the
 // panels of a term (the descriptor's base moves, on the scalar unit), and rows, columns and k past the
 // operand read zero from the descriptor's range check instead of a select. The next panel is in flight in
-// registers while the current one is multiplied from a single LDS buffer (18 KB, 76 VGPRs, six workgroups
-// per CU; a double buffer with one barrier per panel allows four: 172 us against 160 us for stage 1 of a
-// Hubbard bond of 2000 states, 6.3 GFLOP).
+// registers while the current one is multiplied from a single LDS buffer (18 KB; 76 VGPRs, 72 with DOT: six
+// or seven workgroups per CU; a double buffer with one barrier per panel allows four: 172 us against 160 us
+// for stage 1 of a Hubbard bond of 2000 states, 6.3 GFLOP). Now 136 us for that stage (49.6 TFLOP/s executed,
+// the pipe busy 63 % of the time) and 167 us for stage 3, whose 1441 tiles are one uneven round (53 %).
 // AK: A is stored k by k (sa_i 1), else row by row (sa_k 1); B is stored k by k (sb_j 1).
 // DOT: udot[tile] = the sum of its entries times x at their indices in the result vector (butterfly within
 // each wavefront, then the four wavefronts in order).

@@ -12,8 +12,8 @@ typedef double double2_t __attribute__((ext_vector_type(2)));
 constexpr int TK = 16;                       // k-panel
 // A panel in LDS lies in fragment order: entry (16 sub + i, 4 step + q) of a 64 x 16 panel at
 // step T_STEP + (sub / 2) T_PAIR + q T_Q + 2 i + sub % 2, so that one 16-byte read gives a lane its entries
-// of two sub-tiles. The paddings (T_Q 34 for 32, T_STEP 280 for 272) spread the writes of both operand
-// layouts evenly over the banks.
+// of two sub-tiles. The paddings (T_Q 34 for 32, T_STEP 280 for 272) are for the writes of both operand
+// layouts; bank conflicts still take a fifth of a busy CU's cycles.
 constexpr int T_Q = 34, T_PAIR = 4 * T_Q, T_STEP = 2 * T_PAIR + 8, TPANEL = (TK / 4) * T_STEP;
 // an offset past the end of every operand (their extents stay below 2^30 bytes): a load there returns
 // zero and a store is dropped

