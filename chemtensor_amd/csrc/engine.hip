@@ -1377,7 +1377,7 @@ static void build_plain(MatvecPlan& p)
 }
 
 // Plan-time autotuner: every launch form of every stage runs on the plan's own operands (one
-// warm-up and three timed launches, HIP events on the plan stream); the fastest form is kept.
+// warm-up and up to three timed launches, HIP events on the plan stream); the fastest form is kept.
 // time every launch form of each grouped stage on the plan's own descriptors (x = 1, y scratch)
 // and keep the fastest; stage 2 also tries the column-stream form
 void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, bool* use_wapply, bool* use_f12, WTiles* wt, Stage3Split* split3,
@@ -1390,21 +1390,33 @@ void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, 
 	hipEvent_t e0, e1;
 	CTG_HIP(hipEventCreate(&e0));
 	CTG_HIP(hipEventCreate(&e1));
-	auto time3 = [&](const std::function<void()>& f) {
-		f();
+	auto timed = [&](const std::function<void()>& f, int reps) {
 		CTG_HIP(hipEventRecord(e0, s));
-		for (int rep = 0; rep < 3; rep++) f();
+		for (int rep = 0; rep < reps; rep++) f();
 		CTG_HIP(hipEventRecord(e1, s));
 		CTG_HIP(hipEventSynchronize(e1));
 		float ms = 0;
 		CTG_HIP(hipEventElapsedTime(&ms, e0, e1));
-		return ms / 3;
+		return ms / (float)reps;
+	};
+	// a warm-up and three launches; of long stages (50 us) one, and two more unless it took twice the best so far
+	// (the dense forms beside row tiles: molecular operator of 20 orbitals, 512 states, plan 259 against 210 ms)
+	auto time3 = [&](const std::function<void()>& f, float best) {
+		f();
+		if (best > 0.05f && best < 1e30f) {
+			const float ms = timed(f, 1);
+			return ms > 2 * best ? ms : (ms + 2 * timed(f, 2)) / 3;
+		}
+		return timed(f, 3);
 	};
 	// CT_GEMM_LDS overrides the timing-based choice of the LDS-tiled form: 0 never (nor the split stage 3, which
 	// runs on its tiles), 1 the faster of the large tasks and every task, large | all that one where a stage has it
 	const char* lds = getenv("CT_GEMM_LDS");
 	const bool lds_off = lds && lds[0] == '0';
-	float best1 = 1e30f, best2 = 1e30f;
+	// forms of two launches are not timed where one launch takes less than two of any size do (stages of 36
+	// bonds of 36 to 64000 entries: the tiles of the large tasks from 7.8 us, the split stage 3 from 6.1 us)
+	constexpr float TWO_LAUNCHES_MS = 0.006f;
+	float best1 = 1e30f, best2 = 1e30f, rowtiles_ms = 1e30f;
 	for (int st = 0; st < 3; st++) {
 		DevGemm& g = stage[st];
 		GemmBases b = bases[st];
@@ -1412,9 +1424,12 @@ void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, 
 		if (st == 2) b.C = y;
 		float best = 1e30f;
 		int best_form = g.form;
+		// the row tiles first, to which the forms of stage 2 are compared
+		if (st == 1 && wt && wt->ok) rowtiles_ms = time3([&] { launch_wtiles(*wt, *wa, b.B, b.C, s); }, 1e30f);
+		const float known = st == 1 ? rowtiles_ms : 1e30f;
 		for (int f = 0; f < GEMM_NUM_FORMS; f++) {
 			g.form = f;
-			const float ms = time3([&] { launch_grouped_gemm_f64(g, b, s); });
+			const float ms = time3([&] { launch_grouped_gemm_f64(g, b, s); }, std::min(best, known));
 			if (tuned_ms) tuned_ms[st][f] = ms;
 			if (ms < best) { best = ms; best_form = f; }
 		}
@@ -1426,8 +1441,9 @@ void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, 
 			for (const int use : { TILE_LARGE, TILE_ALL }) {
 				if (use == TILE_LARGE ? g.nlitems == 0 : g.naitems == 0) continue;
 				if (lds && strcmp(lds, use == TILE_LARGE ? "all" : "large") == 0) continue;
+				if (!lds && use == TILE_LARGE && best < TWO_LAUNCHES_MS) continue;
 				g.use_lds = use;
-				const float ms = time3([&] { launch_grouped_gemm_f64(g, b, s); });
+				const float ms = time3([&] { launch_grouped_gemm_f64(g, b, s); }, std::min(best, known));
 				if (ms < tile_best) { tile_best = ms; tile_use = use; }
 			}
 			const bool use = tile_use != TILE_NONE && (lds ? !lds_off : tile_best < best);
@@ -1437,9 +1453,13 @@ void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, 
 		if (st == 0) best1 = best;
 		if (st == 1) best2 = best;
 		// after every other allocation of the plan, whose memory it must not take
-		if (st == 2 && split3) split3->upload(s);
+		if (st == 2 && split3) {
+			const char* force = getenv("CT_STAGE3");
+			if (best >= TWO_LAUNCHES_MS || lz_split_saved_ms(nx) > 0 || (force && strcmp(force, "split") == 0)) split3->upload(s);
+			else split3->release();
+		}
 		if (st == 2 && split3 && split3->ok) {
-			const float ms = time3([&] { launch_stage3_units(*split3, b, s); launch_pair_reduce(split3->sum, y, s); });
+			const float ms = time3([&] { launch_stage3_units(*split3, b, s); launch_pair_reduce(split3->sum, y, s); }, best);
 			split3->use = ms < best;
 			split3->use_lanczos = ms - best < lz_split_saved_ms(nx);
 			if (lds_off) split3->use = split3->use_lanczos = false;
@@ -1453,7 +1473,7 @@ void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, 
 	if (use_wapply) {
 		*use_wapply = false;
 		if (wa && wa->ok) {
-			const float ms = time3([&] { launch_wapply(*wa, bases[1].B, bases[1].C, s); });
+			const float ms = time3([&] { launch_wapply(*wa, bases[1].B, bases[1].C, s); }, best2);
 			*use_wapply = ms < best2;
 			if (*use_wapply) best2 = ms;
 			// CT_STAGE2=mfma|stream overrides the timing-based choice
@@ -1463,9 +1483,8 @@ void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, 
 		}
 	}
 	if (wt && wt->ok) {
-		const float ms = time3([&] { launch_wtiles(*wt, *wa, bases[1].B, bases[1].C, s); });
-		wt->use = ms < best2;
-		if (wt->use) best2 = ms;
+		wt->use = rowtiles_ms < best2;
+		if (wt->use) best2 = rowtiles_ms;
 		// CT_STAGE2=mfma|rowtiles overrides the timing-based choice
 		const char* force = getenv("CT_STAGE2");
 		if (force && strcmp(force, "mfma") == 0) wt->use = false;
@@ -1474,7 +1493,7 @@ void autotune_grouped(DevGemm* stage, const GemmBases* bases, const WApply* wa, 
 	if (use_f12) {
 		*use_f12 = false;
 		if (wa && wa->ok && wa->f12_ok) {
-			const float ms = time3([&] { launch_f12(*wa, x, bases[0].B, bases[1].C, s); });
+			const float ms = time3([&] { launch_f12(*wa, x, bases[0].B, bases[1].C, s); }, best1 + best2);
 			*use_f12 = ms < best1 + best2;
 			// CT_STAGE12=fused|separate overrides the timing-based choice
 			const char* force = getenv("CT_STAGE12");

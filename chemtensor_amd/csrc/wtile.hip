@@ -135,31 +135,42 @@ __global__ __launch_bounds__(256, 4) void k_wtile(const WtItem* __restrict__ ite
 // the sets that add the fewest columns to the group (ties: that share the most with it).
 static std::vector<std::vector<int>> greedy_groups(const std::vector<uint64_t>& bits, int count, int nw, int n)
 {
-	std::vector<int> size((size_t)count, 0), rest((size_t)count);
+	std::vector<int> size((size_t)count, 0), rest((size_t)count), add((size_t)count), fresh((size_t)nw);
 	for (int r = 0; r < count; r++) for (int q = 0; q < nw; q++) size[(size_t)r] += __builtin_popcountll(bits[(size_t)r * nw + q]);
 	std::iota(rest.begin(), rest.end(), 0);
 	std::stable_sort(rest.begin(), rest.end(), [&](int x, int y) { return size[(size_t)x] > size[(size_t)y]; });
 	std::vector<std::vector<int>> groups;
 	while (!rest.empty()) {
 		std::vector<int> g;
-		std::vector<uint64_t> u((size_t)nw, 0);
+		std::vector<uint64_t> u((size_t)nw, 0), gain((size_t)nw, 0);
+		for (const int r : rest) add[(size_t)r] = size[(size_t)r];   // columns that r would add to the group
 		size_t best = 0;
 		while ((int)g.size() < n && !rest.empty()) {
 			if (!g.empty()) {
 				int bn = INT32_MAX, bo = -1;
 				for (size_t i = 0; i < rest.size(); i++) {
-					int add = 0;
-					const uint64_t* b = &bits[(size_t)rest[i] * nw];
-					for (int q = 0; q < nw; q++) add += __builtin_popcountll(b[q] & ~u[(size_t)q]);
-					const int overlap = size[(size_t)rest[i]] - add;
-					if (add < bn || (add == bn && overlap > bo)) { bn = add; bo = overlap; best = i; }
+					const int r = rest[i], overlap = size[(size_t)r] - add[(size_t)r];
+					if (add[(size_t)r] < bn || (add[(size_t)r] == bn && overlap > bo)) { bn = add[(size_t)r]; bo = overlap; best = i; }
 				}
 			}
 			const int r = rest[best];
-			for (int q = 0; q < nw; q++) u[(size_t)q] |= bits[(size_t)r * nw + q];
 			g.push_back(r);
 			rest.erase(rest.begin() + (ptrdiff_t)best);
 			best = 0;
+			// the group's new columns (words 'fresh' of 'gain') are none to add any more
+			int nf = 0;
+			for (int q = 0; q < nw; q++) {
+				gain[(size_t)q] = bits[(size_t)r * nw + q] & ~u[(size_t)q];
+				if (gain[(size_t)q]) fresh[(size_t)nf++] = q;
+				u[(size_t)q] |= gain[(size_t)q];
+			}
+			if (nf > 0)
+				for (const int i : rest) {
+					const uint64_t* w = &bits[(size_t)i * nw];
+					int c = 0;
+					for (int k = 0; k < nf; k++) c += __builtin_popcountll(w[fresh[(size_t)k]] & gain[(size_t)fresh[(size_t)k]]);
+					add[(size_t)i] -= c;
+				}
 		}
 		groups.push_back(std::move(g));
 	}
@@ -225,10 +236,17 @@ bool plan_wtiles(WtHost& h, const WApplyHost& wa, const Meta& W, const double* w
 {
 	std::vector<std::vector<WtTile>> tiles(wa.classes.size());
 	std::vector<int64_t> nonzero(wa.classes.size(), 0);
+	std::vector<uint8_t> acts(wa.classes.size(), 0);   // on some block pair
+	for (const int ci : wa.unit_class) acts[(size_t)ci] = 1;
+	// the packs of all columns: address space, of which the packs in use are touched
+	size_t most = 0;
+	for (size_t ci = 0; ci < wa.classes.size(); ci++)
+		if (acts[ci]) most += (size_t)((wa.classes[ci].R + 63) / 64) * (size_t)((wa.classes[ci].K + TK - 1) / TK) * 64 * TK;
+	h.pack.reserve(most);
 	for (size_t ci = 0; ci < wa.classes.size(); ci++) {
 		const WaClass& c = wa.classes[ci];
 		if (c.K > WT_KMAX) return false;
-		if (c.K < 1 || c.R < 1) continue;   // no block pair has it
+		if (!acts[ci] || c.K < 1 || c.R < 1) continue;
 		std::vector<double> m((size_t)c.R * c.K, 0.0);
 		int r0 = 0;
 		for (const auto& mq : c.rows) {
